@@ -16,9 +16,9 @@
 //   prefill_conv_kernel   causal depthwise conv + SiLU over the segment's
 //                         tokens (bf16, the reference's rounding), history
 //                         from the conv ring for tokens before the prompt;
-//                         one more workgroup per chunk computes the gates
-//                         (beta, the cumulative decay G and its exponentials)
-//                         into the chunk's records.
+//                         further workgroups compute the gates (beta, the
+//                         cumulative decay G and its exponentials), a wave
+//                         per head, into the chunk's records.
 //   chunk_prep_kernel     phase A, one workgroup per (chunk, V head):
 //                         l2norm, K K^T and Q K^T on MFMA, blocked fp32
 //                         triangular inverse, U and W on MFMA.
@@ -97,7 +97,8 @@ struct PrefillArgs {
   int num_k_heads;
   int num_v_heads;
   int conv_dim;
-  int x_pairs;  // bf16 x, 4-byte aligned rows: a thread's two channels are one 32-bit load
+  int x_pairs;  // bf16 or fp16 x, 4-byte aligned rows: a thread's two channels are one 32-bit load
+  int conv_cols;  // 512-channel columns of the conv launch; its gate columns follow
   int gate_raw;  // gate_a / gate_b are the raw projections (RIA_GATE_RAW), else g and beta
 };
 
@@ -130,78 +131,88 @@ __device__ __forceinline__ void load8(const float* p, float* v) {
 }
 
 // ---------------------------------------------------------------- conv
-// Two adjacent channels per thread, a tile of 64 tokens per workgroup row.
-// With bf16 inputs every load of the tile is issued at once (one 32-bit load
-// per token for the two channels), then the arithmetic runs: issued in
+// Two adjacent channels per thread, a tile of TT tokens per workgroup row.
+// With bf16 or fp16 inputs every load of the tile is issued at once (one 32-bit
+// load per token for the two channels), then the arithmetic runs: issued in
 // batches, each batch's latency was exposed (187 -> 144 us per 16k-token
-// prompt in one process).  Other input dtypes load tokens in batches of 8.
-// The launch is VALU-bound (the 16k-token prompt moves 0.54 GB, 67 us at
-// 8 TB/s): SiLU takes silu_to_bf16, the same bits as the accurate form at
-// about a third of its instructions, and the bf16 tile path addresses rows
+// prompt in one process).  Rows that are not 4-byte aligned and fp32 inputs
+// load tokens in batches of 8.
+// The launch is VALU-bound on long prompts (the 16k-token prompt moves 0.54
+// GB, 67 us at 8 TB/s): SiLU takes silu_to_bf16, the same bits as the accurate
+// form at about a third of its instructions, and the tile path addresses rows
 // through buffer resources with the row in the scalar offset (146 -> 125 us).
-constexpr int kConvTile = 64;
-static_assert(kConvTile == kChunk, "a conv tile is a chunk: the gate pass takes one per workgroup");
+// A launch of few 64-token tiles leaves too few waves to cover the loads of
+// the next tile with the arithmetic of this one, so it takes tiles of 16
+// (three history rows read per 16): 46.7 -> 36.4 us at 4096 tokens (1024
+// tiles of 64), 36 -> 9.8 us at 300 with the gate pass below; tiles of 64 take
+// 31 us per 4096 tokens in one 16384-token launch, where they stay.
+constexpr int kConvShortTile = 16;
+constexpr int kConvTileWgs = 2048;  // fewer 64-token tiles than this: short tiles
 
-// Gate pass of chunk blockIdx.y (the conv launch's last workgroup column):
-// wave w takes V heads w, w + 4, ..; lane t token t of the chunk.  beta =
+// Gate pass (the conv launch's workgroup columns past the channels): one wave
+// per (chunk cl, V head h), lane t token t of the chunk.  beta =
 // sigmoid(b), g = -exp(A_log) softplus(a + dt_bias) (qwen36_attention_cache.py:
 // 243-247), or both given; G = the sequential cumulative sum of g inside the
 // chunk (tokens past the prompt add 0); then exp(G_t), exp(G_C - G_t) and
 // exp(G_C) for phase A and the scan.  Off phase A's path, where it was a
 // chain of transcendental and dependent adds on one wave (about 15% of an
-// item) while the other three waited at the barrier.
-__device__ __forceinline__ void prefill_gates(const PrefillArgs& a, float* gsh) {
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int cl = blockIdx.y;
+// item) while the other three waited at the barrier.  A chain of two memory
+// round trips and 64 dependent adds: one workgroup per chunk, whose waves
+// walked the heads eight deep, set the launch's time whenever the segment's
+// channels did not (36 us for a 300-token prompt).
+__device__ __forceinline__ void prefill_gates(const PrefillArgs& a, int cl, int h, float* gw) {
+  const int lane = threadIdx.x & 63;
   const int t = (a.chunk0 + cl) * kChunk + lane;
-  const bool ok = t < a.length;
-  float* gw = gsh + wave * kChunk;
-  for (int h = wave; h < a.num_v_heads; h += 4) {
-    float beta = 0.f, g = 0.f;
-    if (ok) {
-      const float ga = a.gate_a[(int64_t)t * a.gate_stride + h], gb = a.gate_b[(int64_t)t * a.gate_stride + h];
-      if (a.gate_raw) {
-        beta = sigmoid_f(gb);
-        g = -expf(a.A_log[h]) * softplus_f(ga + a.dt_bias[h]);
-      } else {
-        beta = gb;
-        g = ga;
-      }
+  float beta = 0.f, g = 0.f;
+  if (t < a.length) {
+    const float ga = a.gate_a[(int64_t)t * a.gate_stride + h], gb = a.gate_b[(int64_t)t * a.gate_stride + h];
+    if (a.gate_raw) {
+      beta = sigmoid_f(gb);
+      g = -expf(a.A_log[h]) * softplus_f(ga + a.dt_bias[h]);
+    } else {
+      beta = gb;
+      g = ga;
     }
-    gw[lane] = g;
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-    // lane t adds g_0 .. g_t one at a time, the order of a sequential cumsum
-    // (the masked terms add +0, which leaves the sum unchanged)
-    float acc = 0.f;
-#pragma unroll
-    for (int i = 0; i < kChunk; i += 4) {
-      const float4 gv = *reinterpret_cast<const float4*>(gw + i);
-      acc += i + 0 <= lane ? gv.x : 0.f;
-      acc += i + 1 <= lane ? gv.y : 0.f;
-      acc += i + 2 <= lane ? gv.z : 0.f;
-      acc += i + 3 <= lane ? gv.w : 0.f;
-    }
-    const float gc = __shfl(acc, kChunk - 1, 64);
-    char* rec = a.rec + ((int64_t)cl * a.num_v_heads + h) * kRecBytes;
-    reinterpret_cast<float4*>(rec + kRecGate)[lane] = float4{beta, acc, expf(acc), expf(gc - acc)};
-    if (lane == 0) *reinterpret_cast<float*>(rec + kRecGl) = expf(gc);
-    __builtin_amdgcn_wave_barrier();  // gw is read by every lane before the next head writes it
   }
+  gw[lane] = g;
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+  // lane t adds g_0 .. g_t one at a time, the order of a sequential cumsum
+  // (the masked terms add +0, which leaves the sum unchanged)
+  float acc = 0.f;
+#pragma unroll
+  for (int i = 0; i < kChunk; i += 4) {
+    const float4 gv = *reinterpret_cast<const float4*>(gw + i);
+    acc += i + 0 <= lane ? gv.x : 0.f;
+    acc += i + 1 <= lane ? gv.y : 0.f;
+    acc += i + 2 <= lane ? gv.z : 0.f;
+    acc += i + 3 <= lane ? gv.w : 0.f;
+  }
+  const float gc = __shfl(acc, kChunk - 1, 64);
+  char* rec = a.rec + ((int64_t)cl * a.num_v_heads + h) * kRecBytes;
+  reinterpret_cast<float4*>(rec + kRecGate)[lane] = float4{beta, acc, expf(acc), expf(gc - acc)};
+  if (lane == 0) *reinterpret_cast<float*>(rec + kRecGl) = expf(gc);
 }
 
-template <int XT>
+// Grid x: a.conv_cols columns of 512 channels, then the gate columns; y: the
+// segment's tiles, TT tokens each, whole chunks of them (tiles past the last
+// token exit).
+template <int XT, int TT>
 __global__ __launch_bounds__(256) void prefill_conv_kernel(PrefillArgs a) {
-  if (blockIdx.x == gridDim.x - 1) {
+  constexpr int kTiles = kChunk / TT;  // tiles of a chunk: they share its gate workgroups
+  static_assert(kChunk % TT == 0, "a chunk is whole tiles");
+  if (static_cast<int>(blockIdx.x) >= a.conv_cols) {
     __shared__ __attribute__((aligned(16))) float gsh[4 * kChunk];
-    prefill_gates(a, gsh);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int h = 4 * ((blockIdx.x - a.conv_cols) * kTiles + blockIdx.y % kTiles) + wave;
+    if (h < a.num_v_heads) prefill_gates(a, blockIdx.y / kTiles, h, gsh + wave * kChunk);
     return;
   }
   const int c = 2 * (blockIdx.x * 256 + threadIdx.x);
-  if (c >= a.conv_dim) return;
-  const int t_begin = a.tok0 + blockIdx.y * kConvTile;
-  const int t_end = min(t_begin + kConvTile, a.tok0 + a.seg_tokens);
+  const int t_begin = a.tok0 + blockIdx.y * TT;
+  const int t_end = min(t_begin + TT, a.tok0 + a.seg_tokens);
+  if (c >= a.conv_dim || t_begin >= t_end) return;
   const uint4 wv = *reinterpret_cast<const uint4*>(a.conv_w + (int64_t)c * kConvTaps);  // 2 channels x 4 taps
   const float wa[4] = {bf16_bits_to_f32(wv.x & 0xffffu), bf16_bits_to_f32(wv.x >> 16),
                        bf16_bits_to_f32(wv.y & 0xffffu), bf16_bits_to_f32(wv.y >> 16)};
@@ -235,7 +246,7 @@ __global__ __launch_bounds__(256) void prefill_conv_kernel(PrefillArgs a) {
     hb[0] = hb[1]; hb[1] = hb[2]; hb[2] = xb;
     return B16::pack2(silu_to_bf16(B16::lo_f32(r)), silu_to_bf16(B16::hi_f32(r)));
   };
-  if (XT == RIA_DT_BF16 && a.x_pairs) {
+  if (XT != RIA_DT_F32 && a.x_pairs) {
     // Every load of the tile at once.  Buffer resources over the tile's rows
     // take the row in the scalar offset, so no per-token address arithmetic
     // (x rows clamped to the segment; x_stride < 2^24 elements).
@@ -246,15 +257,20 @@ __global__ __launch_bounds__(256) void prefill_conv_kernel(PrefillArgs a) {
     const auto ps = __builtin_amdgcn_make_buffer_rsrc(a.post + (int64_t)(t_begin - a.tok0) * a.conv_dim, 0,
                                                       rows * a.conv_dim * 2, kBufferWord3);
     const int voff = c * 2;
-    uint32_t xr[kConvTile];
+    uint32_t xr[TT];
 #pragma unroll
-    for (int u = 0; u < kConvTile; ++u)
+    for (int u = 0; u < TT; ++u)
       xr[u] = __builtin_amdgcn_raw_buffer_load_b32(xs, voff, min(u, rows - 1) * (int)a.x_stride * 2, 0);
+    auto as_bf16 = [](uint32_t w) -> uint32_t {  // the token's two values as bf16
+      if constexpr (XT == RIA_DT_F16) return B16::pack2(Kv16<RIA_DT_F16>::lo_f32(w), Kv16<RIA_DT_F16>::hi_f32(w));
+      return w;
+    };
 #pragma unroll
-    for (int u = 0; u < kConvTile; ++u)
-      if (u < rows)
-        __builtin_amdgcn_raw_buffer_store_b32(step(B16::lo_f32(xr[u]), B16::hi_f32(xr[u])), ps, voff,
-                                              u * a.conv_dim * 2, 0);
+    for (int u = 0; u < TT; ++u)
+      if (u < rows) {
+        const uint32_t w = as_bf16(xr[u]);
+        __builtin_amdgcn_raw_buffer_store_b32(step(B16::lo_f32(w), B16::hi_f32(w)), ps, voff, u * a.conv_dim * 2, 0);
+      }
   } else {
     for (int tb = t_begin; tb < t_end; tb += 8) {
       float xa[8], xb[8];
@@ -1034,7 +1050,7 @@ extern "C" int ria_gdn_prefill(int length, int num_k_heads, int num_v_heads, con
   PrefillArgs a{};
   a.x = mixed_qkv;
   a.x_stride = x_row_stride;
-  a.x_pairs = x_dtype == RIA_DT_BF16 && reinterpret_cast<uintptr_t>(mixed_qkv) % 4 == 0 && x_row_stride % 2 == 0 &&
+  a.x_pairs = x_dtype != RIA_DT_F32 && reinterpret_cast<uintptr_t>(mixed_qkv) % 4 == 0 && x_row_stride % 2 == 0 &&
               x_row_stride < (int64_t(1) << 24);
   a.conv_w = static_cast<const uint16_t*>(conv_weight);
   a.conv_ring = static_cast<uint16_t*>(conv_ring);
@@ -1062,11 +1078,17 @@ extern "C" int ria_gdn_prefill(int length, int num_k_heads, int num_v_heads, con
     a.seg_chunks = min(seg_chunks, total_chunks - c0);
     a.tok0 = c0 * kChunk;
     a.seg_tokens = min(a.seg_chunks * kChunk, length - a.tok0);
-    dim3 cgrid((conv_dim / 2 + 255) / 256 + 1, (a.seg_tokens + kConvTile - 1) / kConvTile);  // + the gate pass
+    a.conv_cols = (conv_dim / 2 + 255) / 256;
+    const bool short_tiles = a.conv_cols * a.seg_chunks < kConvTileWgs;
+    const int tiles = short_tiles ? kChunk / kConvShortTile : 1;  // per chunk
+    dim3 cgrid(a.conv_cols + ((num_v_heads + 3) / 4 + tiles - 1) / tiles, a.seg_chunks * tiles);
     dim3 pgrid(num_v_heads, a.seg_chunks);
     dim3 sgrid(num_v_heads * (kDim / 16));
 #define RIA_PREFILL_PHASES(XT_)                                                                          \
-  hipLaunchKernelGGL((prefill_conv_kernel<XT_>), cgrid, dim3(256), 0, st, a);                           \
+  if (short_tiles)                                                                                       \
+    hipLaunchKernelGGL((prefill_conv_kernel<XT_, kConvShortTile>), cgrid, dim3(256), 0, st, a);          \
+  else                                                                                                   \
+    hipLaunchKernelGGL((prefill_conv_kernel<XT_, kChunk>), cgrid, dim3(256), 0, st, a);                  \
   hipLaunchKernelGGL((chunk_prep_kernel<XT_>), pgrid, dim3(256), 0, st, a)
     if (x_dtype == RIA_DT_BF16) {
       RIA_PREFILL_PHASES(RIA_DT_BF16);

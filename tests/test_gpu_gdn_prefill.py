@@ -202,3 +202,27 @@ def test_prefill_conv_load_paths_agree(gpu):
     want, s_want, _ = _oracle_tokens(params, inputs, length, state0[None], ring_to_window(ring0, 5))
     assert_act_close(res[0][0], want, "outputs vs oracle")
     assert_state_close(res[0][1][None], s_want, "final state vs oracle")
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("length", [15, 16, 17, 79, 129])
+def test_prefill_conv_short_tiles(gpu, dtype, length):
+    """Prompts that end around the conv's 16-token tiles and inside a chunk:
+    16-bit rows loaded in pairs against the per-channel path (odd row stride),
+    the same bits, and the oracle on the same 16-bit inputs."""
+    announce(f"gdn_prefill: {dtype} conv tiles, {length} tokens")
+    params = W.gdn_layer_params(61)
+    inputs = W.gdn_step_inputs(62, length, 1)
+    inputs["mixed"] = inputs["mixed"].to(dtype)
+    state0, ring0 = _init(63)
+    mixed = inputs["mixed"][:length, 0]
+    wide = torch.zeros((length, W.CONV_DIM + 1), dtype=dtype)
+    wide[:, :W.CONV_DIM] = mixed
+    got = _gpu_prefill(gpu, params, inputs, length, state0, ring0, 6)
+    inputs["mixed"] = wide.to(gpu)[:, None, :W.CONV_DIM]
+    odd = _gpu_prefill(gpu, params, inputs, length, state0, ring0, 6)
+    assert all(torch.equal(x, y) for x, y in zip(got, odd))
+    inputs["mixed"] = mixed[:, None].float()
+    want, s_want, _ = _oracle_tokens(params, inputs, length, state0[None], ring_to_window(ring0, 6))
+    assert_act_close(got[0], want, "outputs vs oracle")
+    assert_state_close(got[1][None], s_want, "final state vs oracle")
