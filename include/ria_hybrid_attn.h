@@ -442,6 +442,31 @@ int ria_attn_prefill_staged(int length, int num_q_heads, int num_kv_heads,
                             void* out, int phase, void* stream);
 
 /*
+ * ria_attn_prefill_staged (`stage` may be null) with a workspace that lets the
+ * attention launch split the keys of a query block between workgroups when
+ * the prompt has too few query blocks to fill the GPU; a further launch merges
+ * the pieces.  ria_attn_prefill_workspace_bytes gives the bytes of the split
+ * chosen for a prompt (0: not split; fp16_keys: nonzero when the attention
+ * reads fp16 keys, from the stage or an fp16 cache).  A workspace (16-byte
+ * aligned) that is null or smaller runs unsplit.  The pages are those of
+ * ria_attn_prefill_phase bit for bit, the outputs equal up to the order of the
+ * fp32 sums.
+ */
+int64_t ria_attn_prefill_workspace_bytes(int length, int num_q_heads, int num_kv_heads, int32_t start_pos,
+                                         int fp16_keys);
+int ria_attn_prefill_split(int length, int num_q_heads, int num_kv_heads,
+                           const void* q, int64_t q_row_stride,
+                           const void* k, int64_t k_row_stride,
+                           const void* v, int64_t v_row_stride,
+                           const void* gate, int64_t gate_row_stride, int act_dtype,
+                           void* k_cache, void* v_cache, int kv_dtype, int num_pages,
+                           const int32_t* page_table_row, int64_t page_capacity, int32_t start_pos,
+                           const float* inv_freq, int rope_dim,
+                           const float* q_norm_weight, const float* k_norm_weight, float scale,
+                           void* stage, int64_t stage_bytes, void* workspace, int64_t workspace_bytes,
+                           void* out, int phase, void* stream);
+
+/*
  * Split size ria_attn_decode would choose for these context lengths (a host
  * array of `batch` tokens-attended counts): long splits, down to one page
  * per wave when the batch holds too few pages to occupy the GPU.  Passing

@@ -31,6 +31,7 @@
 //   * the gated result leaves through LDS so the output stores are coalesced;
 //   * query blocks are scheduled from the last (most keys) to the first.
 #include <math.h>
+#include <algorithm>
 
 #include "ria_common.h"
 
@@ -50,6 +51,8 @@ constexpr int kPrefillWaves = 8;                   // one query head per wave
 constexpr int kPrefillThreads = 64 * kPrefillWaves;
 constexpr int kStagePitch = kAttnHeadDim + 4;      // floats per staged output row
 constexpr int kPrefillLds = kPrefillWaves * 16 * kStagePitch * 4;  // output stage; the ring (128 KiB) aliases it
+constexpr int kMaxPieces = 32;      // pieces of a query block's keys
+constexpr int kMinPieceBlocks = 4;  // 32-key blocks of a piece: two refills of the ring
 static_assert(kRingSlots * kSlotVec * 16 <= kPrefillLds, "ring must fit in the LDS block");
 
 struct PrefillAttnArgs {
@@ -72,7 +75,25 @@ struct PrefillAttnArgs {
   int group;
   void* out;
   int staged;  // keys from an fp16 stage with tile (page p, KV head) at p * Hkv + kvh, not the page table
+  int chunk;   // 32-key blocks per piece of a query block's keys (even); 0: no query block is split
+  float* part;     // split pieces: unnormalised O, [piece][head of the group][token 16][256]
+  float2* part_ml;  // .. and the columns' (max, sum), [piece][head of the group][token 16]
 };
+
+// Pieces.  The keys of a query block are split every `chunk` 32-key blocks,
+// as far as a piece's first key is visible to the block's first query (so
+// every column of every piece has a finite max); the last piece takes the
+// rest.  Piece s exists for the query blocks qb >= first_query_block(s).  A
+// launch lists the pieces by s, each s from the last query block down, and
+// both kernels find a piece's index by the same counts.
+__host__ __device__ inline int first_query_block(int s, int chunk, int start, int nqb) {
+  if (s == 0) return 0;
+  const int64_t k0 = (int64_t)s * chunk * 32 - start;  // query tokens from here on see the piece's first key
+  return k0 <= 0 ? 0 : static_cast<int>(k0 + 15 < (int64_t)16 * nqb ? (k0 + 15) / 16 : nqb);
+}
+__host__ __device__ inline int query_block_pieces(int qb, int chunk, int start) {
+  return chunk ? 1 + (start + 16 * qb) / (32 * chunk) : 1;
+}
 
 // Key held by row r (0..15) of score tile m (0, 1) of a 32-key block, as
 // (page of the block, token): lane group g = r / 4 of both tiles together
@@ -109,8 +130,12 @@ __global__ __launch_bounds__(kPrefillThreads) __attribute__((amdgpu_waves_per_eu
   // keep 11 significant bits in the hi part alone, which is enough here
   constexpr bool kSplit = KVT == RIA_DT_BF16;
   const int nqb = (a.length + 15) / 16;
-  const int qb = nqb - 1 - static_cast<int>(blockIdx.x) / a.num_kv_heads;  // heaviest blocks first
-  const int kvh = static_cast<int>(blockIdx.x) % a.num_kv_heads;
+  int piece = 0, unit = static_cast<int>(blockIdx.x);
+  if (a.chunk)
+    for (int n; unit >= (n = (nqb - first_query_block(piece, a.chunk, a.start, nqb)) * a.num_kv_heads); unit -= n) ++piece;
+  const int qb = nqb - 1 - unit / a.num_kv_heads;  // heaviest blocks first
+  const int kvh = unit % a.num_kv_heads;
+  const int pieces = query_block_pieces(qb, a.chunk, a.start);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int n = lane & 15;   // MFMA column (token 16 qb + n) / row (key or dim)
   const int g4 = lane >> 4;  // lane group: k slice of the operands, row group of the results
@@ -218,7 +243,8 @@ __global__ __launch_bounds__(kPrefillThreads) __attribute__((amdgpu_waves_per_eu
 
   const int q_last = a.start + min(16 * qb + 15, a.length - 1);  // last query position of the block
   const int npages = q_last / kPageTokens + 1;                   // <= pt_len (checked on the host)
-  const int nblk = (npages + 1) / 2;
+  const int blk0 = piece * a.chunk;  // this piece's key blocks: blk0 (even) .. nblk - 1
+  const int nblk = piece + 1 < pieces ? blk0 + a.chunk : (npages + 1) / 2;
   const int kmax = min(q_last, ctx_total - 1);  // last key any column of the block uses
   const int q_first = a.start + 16 * qb;         // first query position of the block
 
@@ -337,8 +363,8 @@ __global__ __launch_bounds__(kPrefillThreads) __attribute__((amdgpu_waves_per_eu
     }
     if (__any(mloc > m_run + 8.0f)) {
       const float mx = swap_max(swap_max(mloc, true), false);
-      // m_run is finite from the first block on (key 0 is visible to every
-      // column), so masked scores give exp2(-inf) = 0
+      // m_run is finite from the first block on (the piece's first key is
+      // visible to every column), so masked scores give exp2(-inf) = 0
       const bool grow = mx > m_run + 8.0f;
       const float m_new = grow ? mx : m_run;
       const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);  // 0 on the first block, where o and l are 0
@@ -372,9 +398,9 @@ __global__ __launch_bounds__(kPrefillThreads) __attribute__((amdgpu_waves_per_eu
   // direct-to-LDS copies, only on each being written to LDS when the counter
   // no longer holds it; pairing gives each copy two iterations to land.
   f32x4 sc[2];
-  issue(0);
-  if (nblk > 1) issue(1);
-  for (int b = 0; b < nblk; ++b) {
+  issue(blk0);
+  if (blk0 + 1 < nblk) issue(blk0 + 1);
+  for (int b = blk0; b < nblk; ++b) {
     if ((b & 1) == 0) {
       asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
       if (b + 2 < nblk) issue(b + 2);
@@ -407,6 +433,15 @@ __global__ __launch_bounds__(kPrefillThreads) __attribute__((amdgpu_waves_per_eu
     softmax_pv(b, sc);
   }
 
+  if (pieces > 1) {  // a split query block: the combine launch merges the pieces
+    if (!head_ok) return;
+    const int64_t row = ((int64_t)blockIdx.x * a.group + wave) * 16 + n;
+    float* pp = a.part + row * kAttnHeadDim + 4 * g4;
+#pragma unroll
+    for (int dt = 0; dt < 16; ++dt) *reinterpret_cast<f32x4*>(pp + 16 * dt) = o[dt];
+    if (g4 == 0) a.part_ml[row] = float2{m_run, o[16][0]};
+    return;
+  }
   // ---- normalise, stage (the ring is dead once every wave has left the loop), gate, store
   lds_barrier();
   const float l_tot = o[16][0];
@@ -434,12 +469,121 @@ __global__ __launch_bounds__(kPrefillThreads) __attribute__((amdgpu_waves_per_eu
   }
 }
 
+// Merges the pieces of every split query block: one wave per (token, query
+// head), lane l dims 4 l .. + 3.  out = sum_s w_s O_s / sum_s w_s l_s * sigmoid(gate),
+// w_s = 2^(m_s - max m).  Bound by the partials' bytes (16 tokens x 8 heads x
+// 1 KB per piece, written and read once).
+template <int AT>
+__global__ __launch_bounds__(256) void attn_prefill_combine_kernel(PrefillAttnArgs a) {
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t r = (int64_t)blockIdx.x * 4 + wave;
+  const int t = static_cast<int>(r / a.num_q_heads), head = static_cast<int>(r % a.num_q_heads);
+  if (t >= a.length) return;
+  const int nqb = (a.length + 15) / 16, qb = t / 16;
+  const int pieces = query_block_pieces(qb, a.chunk, a.start);
+  if (pieces == 1) return;  // its workgroup stored the result
+  const int d = 4 * lane;
+  float g[4], y[4];
+  load_act4<AT>(a.gate, (int64_t)t * a.gate_stride + (int64_t)head * kAttnHeadDim + d, g);
+  const int kvh = head / a.group;
+  // row of piece s in the partials: its index in the launch, this head and token
+  auto row_of = [&](int s, int64_t before) {
+    return ((before + (int64_t)(nqb - 1 - qb) * a.num_kv_heads + kvh) * a.group + head % a.group) * 16 + t % 16;
+  };
+  int64_t before = 0;
+  float m = -INFINITY, l = 0.f;
+  f32x4 o = {0.f, 0.f, 0.f, 0.f};
+  for (int s0 = 0; s0 < pieces; s0 += 4) {  // four pieces' loads in flight
+    float2 ml[4];
+    f32x4 po[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int s = min(s0 + j, pieces - 1);
+      const int64_t row = row_of(s, before);
+      ml[j] = a.part_ml[row];
+      po[j] = *reinterpret_cast<const f32x4*>(a.part + row * kAttnHeadDim + d);
+      if (s0 + j + 1 < pieces) before += (int64_t)(nqb - first_query_block(s, a.chunk, a.start, nqb)) * a.num_kv_heads;
+    }
+    float mx = m;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) mx = fmaxf(mx, ml[j].x);
+    const float keep = __builtin_amdgcn_exp2f(m - mx);
+    o *= keep;
+    l *= keep;
+    m = mx;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (s0 + j < pieces) {
+        const float w = __builtin_amdgcn_exp2f(ml[j].x - mx);
+        o += po[j] * w;
+        l = fmaf(ml[j].y, w, l);
+      }
+  }
+  const float inv = 1.0f / l;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float x = o[i] * inv;
+    y[i] = AT == RIA_DT_BF16 ? gate_mul_to_bf16(x, g[i]) : mul_rn(x, sigmoid_f(g[i]));
+  }
+  store_act4<AT>(a.out, ((int64_t)t * a.num_q_heads + head) * kAttnHeadDim + d, y);
+}
+
 template <int AT>
 static void launch_prefill(const PrefillAttnArgs& a, const int32_t* pt, int kv_dtype, dim3 grid, hipStream_t st) {
   if (kv_dtype == RIA_DT_F16)
     hipLaunchKernelGGL((attn_prefill_kernel<AT, RIA_DT_F16>), grid, dim3(kPrefillThreads), 0, st, a, pt);
   else
     hipLaunchKernelGGL((attn_prefill_kernel<AT, RIA_DT_BF16>), grid, dim3(kPrefillThreads), 0, st, a, pt);
+  if (a.chunk) {
+    const int64_t rows = (int64_t)a.length * a.num_q_heads;
+    hipLaunchKernelGGL((attn_prefill_combine_kernel<AT>), dim3(static_cast<unsigned>((rows + 3) / 4)), dim3(256), 0, st, a);
+  }
+}
+
+// How a prompt's query blocks are split (PrefillAttnArgs::chunk) and the
+// pieces that makes.  One workgroup per CU runs at a time, so the launch
+// takes about max(longest piece, work / CUs): a prompt whose query blocks
+// number fewer than the CUs, or whose last blocks hold most keys, is cut into
+// pieces until the cut costs more (the prologue of each piece, the partials'
+// traffic, the combine launch) than it evens out.  Costs in key blocks of the
+// fp16 kernel (about 1 us each), from kernel times on MI355X: prologue and
+// epilogue of a whole query block 16, of a piece 9; a bf16 block (hi + lo
+// operands) 1.5; combine 6 + one per 15 pieces.
+struct PrefillPlan {
+  int chunk;       // 0: unsplit
+  int64_t pieces;  // workgroups of the launch
+};
+static PrefillPlan plan_prefill(int length, int start, int num_kv_heads, bool fp16_keys) {
+  const int cus = device_cus(), nqb = (length + 15) / 16;
+  const int most = ((start + length - 1) / kPageTokens + 2) / 2;  // key blocks of the last query block
+  const double per_block = fp16_keys ? 1.0 : 1.5;
+  PrefillPlan best{0, (int64_t)nqb * num_kv_heads};
+  double best_cost = -1;
+  for (int k = 1; k <= kMaxPieces; ++k) {
+    const int chunk = k == 1 ? 0 : ((most + k - 1) / k + 1) / 2 * 2;
+    if (k > 1 && chunk < kMinPieceBlocks) break;
+    int64_t pieces = 0;
+    for (int s = 0; s < k; ++s) pieces += (int64_t)(nqb - first_query_block(s, chunk, start, nqb)) * num_kv_heads;
+    // key blocks in all: query block qb has (start + 16 qb) / 32 + 1 of them
+    const double work = (double)num_kv_heads * nqb * ((start + 8.0 * nqb) / 32 + 1) * per_block + pieces * (k == 1 ? 16.0 : 9.0);
+    const double longest = (k == 1 ? most : chunk + 1) * per_block + (k == 1 ? 16.0 : 9.0);
+    double cost = std::max(longest, work / cus);
+    if (k > 1) {  // whole query blocks run longest first and end together; pieces of several sizes do not
+      if (pieces > 2 * cus) continue;
+      if (pieces > cus) cost = std::max(cost, work / cus + longest / 2);
+      cost += 6.0 + pieces / 15.0;
+    }
+    if (best_cost < 0 || cost < best_cost) {
+      best_cost = cost;
+      best = PrefillPlan{chunk, pieces};
+    }
+  }
+  return best;
+}
+
+static int64_t partial_bytes(const PrefillPlan& p, int group) {
+  return p.chunk ? p.pieces * group * 16 * (int64_t)(kAttnHeadDim * sizeof(float) + sizeof(float2)) : 0;
 }
 
 }  // namespace ria
@@ -464,7 +608,8 @@ static int prefill_impl(int length, int num_q_heads, int num_kv_heads, const voi
                         int64_t gate_row_stride, int act_dtype, void* k_cache, void* v_cache, int kv_dtype,
                         int num_pages, const int32_t* page_table_row, int64_t page_capacity, int32_t start_pos,
                         const float* inv_freq, int rope_dim, const float* q_norm_weight, const float* k_norm_weight,
-                        float scale, void* stage, int64_t stage_bytes, void* out, int phase, void* stream) {
+                        float scale, void* stage, int64_t stage_bytes, void* workspace, int64_t workspace_bytes,
+                        void* out, int phase, void* stream) {
   if (phase < RIA_PREFILL_APPEND || phase > RIA_PREFILL_BOTH)
     return set_error(RIA_ERR_INVALID, "ria_attn_prefill: phase must be 1 (append), 2 (attention) or 3 (both)");
   if (length < 0 || start_pos < 0) return set_error(RIA_ERR_INVALID, "ria_attn_prefill: negative length or start");
@@ -542,6 +687,17 @@ static int prefill_impl(int length, int num_q_heads, int num_kv_heads, const voi
     key_dtype = RIA_DT_F16;
   }
   dim3 grid(static_cast<unsigned>(blocks));
+  if (workspace) {
+    if (reinterpret_cast<uintptr_t>(workspace) % 16)
+      return set_error(RIA_ERR_INVALID, "ria_attn_prefill: workspace must be 16-byte aligned");
+    const PrefillPlan plan = plan_prefill(length, start_pos, num_kv_heads, key_dtype == RIA_DT_F16);
+    if (plan.chunk && partial_bytes(plan, group) <= workspace_bytes) {  // a smaller workspace: no split
+      a.chunk = plan.chunk;
+      a.part = static_cast<float*>(workspace);
+      a.part_ml = reinterpret_cast<float2*>(a.part + plan.pieces * group * 16 * kAttnHeadDim);
+      grid.x = static_cast<unsigned>(plan.pieces);
+    }
+  }
   hipStream_t st = static_cast<hipStream_t>(stream);
   if (act_dtype == RIA_DT_BF16)
     launch_prefill<RIA_DT_BF16>(a, page_table_row, key_dtype, grid, st);
@@ -564,7 +720,7 @@ extern "C" int ria_attn_prefill_phase(int length, int num_q_heads, int num_kv_he
   return prefill_impl(length, num_q_heads, num_kv_heads, q, q_row_stride, k, k_row_stride, v, v_row_stride, gate,
                       gate_row_stride, act_dtype, k_cache, v_cache, kv_dtype, num_pages, page_table_row,
                       page_capacity, start_pos, inv_freq, rope_dim, q_norm_weight, k_norm_weight, scale, nullptr, 0,
-                      out, phase, stream);
+                      nullptr, 0, out, phase, stream);
 }
 
 extern "C" int64_t ria_attn_prefill_stage_bytes(int length, int num_kv_heads) {
@@ -584,7 +740,27 @@ extern "C" int ria_attn_prefill_staged(int length, int num_q_heads, int num_kv_h
   return prefill_impl(length, num_q_heads, num_kv_heads, q, q_row_stride, k, k_row_stride, v, v_row_stride, gate,
                       gate_row_stride, act_dtype, k_cache, v_cache, kv_dtype, num_pages, page_table_row,
                       page_capacity, start_pos, inv_freq, rope_dim, q_norm_weight, k_norm_weight, scale, stage,
-                      stage_bytes, out, phase, stream);
+                      stage_bytes, nullptr, 0, out, phase, stream);
+}
+
+extern "C" int64_t ria_attn_prefill_workspace_bytes(int length, int num_q_heads, int num_kv_heads, int32_t start_pos,
+                                                    int fp16_keys) {
+  if (length <= 0 || start_pos < 0 || num_kv_heads <= 0 || num_q_heads <= 0 || num_q_heads % num_kv_heads) return 0;
+  return partial_bytes(plan_prefill(length, start_pos, num_kv_heads, fp16_keys != 0), num_q_heads / num_kv_heads);
+}
+
+extern "C" int ria_attn_prefill_split(int length, int num_q_heads, int num_kv_heads, const void* q,
+                                      int64_t q_row_stride, const void* k, int64_t k_row_stride, const void* v,
+                                      int64_t v_row_stride, const void* gate, int64_t gate_row_stride, int act_dtype,
+                                      void* k_cache, void* v_cache, int kv_dtype, int num_pages,
+                                      const int32_t* page_table_row, int64_t page_capacity, int32_t start_pos,
+                                      const float* inv_freq, int rope_dim, const float* q_norm_weight,
+                                      const float* k_norm_weight, float scale, void* stage, int64_t stage_bytes,
+                                      void* workspace, int64_t workspace_bytes, void* out, int phase, void* stream) {
+  return prefill_impl(length, num_q_heads, num_kv_heads, q, q_row_stride, k, k_row_stride, v, v_row_stride, gate,
+                      gate_row_stride, act_dtype, k_cache, v_cache, kv_dtype, num_pages, page_table_row,
+                      page_capacity, start_pos, inv_freq, rope_dim, q_norm_weight, k_norm_weight, scale, stage,
+                      stage_bytes, workspace, workspace_bytes, out, phase, stream);
 }
 
 extern "C" int ria_attn_prefill(int length, int num_q_heads, int num_kv_heads, const void* q, int64_t q_row_stride,

@@ -897,14 +897,6 @@ static void launch_ks(const LinearArgs& a, KsShape s, dim3 grid, hipStream_t st)
     launch_ks_k<2, 2, 6, XB>(a, grid, st);
 }
 
-static int device_cus() {
-  int dev = 0, cus = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
-    cus = 256;
-  return cus;
-}
-
 static bool lin_dtype_ok(int dt) { return dt == RIA_DT_BF16 || dt == RIA_DT_F16 || dt == RIA_DT_F32; }
 
 }  // namespace ria

@@ -400,4 +400,13 @@ __device__ __forceinline__ float half_wave_sum(float v) {
 namespace ria {
 int set_error(int code, const char* fmt, ...);
 int check_launch(const char* what);
+// Compute units of the current device.
+inline int device_cus() {
+  int dev = 0, cus = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
+    cus = 256;
+  return cus;
+}
+
 }  // namespace ria

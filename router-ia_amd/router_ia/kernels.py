@@ -1048,6 +1048,7 @@ def attn_prefill(
     q_norm_weight: torch.Tensor | None = None,
     k_norm_weight: torch.Tensor | None = None,
     stage: torch.Tensor | None = None,
+    workspace: torch.Tensor | None = None,
 ) -> torch.Tensor:
     """Causal GQA prefill of one sequence's prompt over its paged cache (ria_attn_prefill_phase).
 
@@ -1059,7 +1060,9 @@ def attn_prefill(
     uint8 device tensor of at least prefill_stage_bytes(L, Hkv); both phases
     take the same one) a prompt that starts the sequence (start 0) is
     attended over fp16 copies of its own keys and values
-    (ria_attn_prefill_staged).
+    (ria_attn_prefill_staged).  With a ``workspace`` (uint8, at least
+    prefill_attn_workspace_bytes) the keys of a short prompt's query blocks
+    are split between workgroups (ria_attn_prefill_split).
     """
     length = int(q.shape[0])
     num_q_heads = int(q.shape[1])
@@ -1088,16 +1091,24 @@ def attn_prefill(
             _ptr(k_cache), _ptr(v_cache), dtype_code(k_cache), pages, _ptr(page_table), cap, int(start),
             _ptr(inv_freq), rope_dim, _norm_weight("q_norm_weight", q_norm_weight, ATTN_HEAD_DIM, dev),
             _norm_weight("k_norm_weight", k_norm_weight, ATTN_HEAD_DIM, dev), float(scale))
-    if stage is None:
+    for name, t in (("stage", stage), ("workspace", workspace)):
+        _require_gpu(name, t, dev)
+        if t is not None and not t.is_contiguous():
+            raise ValueError(f"{name} must be contiguous")
+    if stage is None and workspace is None:
         rc = nat.load().ria_attn_prefill_phase(*head, _ptr(out), int(phase), _stream(dev))
     else:
-        _require_gpu("stage", stage, dev)
-        if not stage.is_contiguous():
-            raise ValueError("stage must be contiguous")
-        rc = nat.load().ria_attn_prefill_staged(*head, _ptr(stage), stage.numel() * stage.element_size(), _ptr(out),
-                                                int(phase), _stream(dev))
+        rc = nat.load().ria_attn_prefill_split(*head, _ptr(stage), 0 if stage is None else stage.nbytes,
+                                               _ptr(workspace), 0 if workspace is None else workspace.nbytes,
+                                               _ptr(out), int(phase), _stream(dev))
     nat.check(rc, "ria_attn_prefill")
     return out
+
+
+def prefill_attn_workspace_bytes(length: int, num_q_heads: int, num_kv_heads: int, start: int, fp16_keys: bool) -> int:
+    """Bytes of the split attn_prefill makes of a prompt's keys (ria_attn_prefill_workspace_bytes; 0: none)."""
+    return int(nat.load().ria_attn_prefill_workspace_bytes(int(length), int(num_q_heads), int(num_kv_heads),
+                                                           int(start), int(fp16_keys)))
 
 
 def prefill_stage_bytes(length: int, num_kv_heads: int) -> int:

@@ -211,3 +211,35 @@ def test_attn_prefill_keeps_its_tolerance_margin(gpu, staged, bound):
             worst = max(worst, ratio)
     print(f"worst error / tolerance: {worst:.3f}", flush=True)
     assert worst <= bound, f"worst error is {worst:.3f} of the tolerance"
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("length,start,hq,hkv", [(1, 300, 16, 2), (17, 2047, 16, 2), (100, 1000, 6, 2),
+                                                  (333, 0, 16, 2), (500, 2100, 16, 2), (1000, 0, 16, 2), (130, 513, 4, 4)])
+def test_attn_prefill_split_keys(gpu, length, start, hq, hkv):
+    """Query blocks whose keys are split between workgroups against the unsplit
+    launch, fp32 activations.  Both round the probabilities (fp16: 2^-11,
+    bf16 hi + lo: 2^-16 relative, about different maxima) in products and
+    normaliser alike, so each output moves at most 2 * 2 * u * max |v|."""
+    announce(f"attn_prefill split: {length} after {start}, Hq={hq}, Hkv={hkv}")
+    _, k0, v0, _ = _inputs(7, max(start, 1), hq, hkv, torch.float32)
+    q, k, v, gate = _inputs(8 + length, length, hq, hkv, torch.float32)
+    inv = rope_inv_freq(10_000_000.0, 64).to(gpu)
+    for kv_dtype, staged in ((torch.bfloat16, start == 0), (torch.float16, False)):
+        kv = _cache(gpu, start + length, hkv, kv_dtype)
+        if start:
+            K.kv_append_seq(k0.to(gpu), v0.to(gpu), kv.k[0], kv.v[0], kv.page_table[0], start=0, inv_freq=inv)
+        fp16 = staged or kv_dtype == torch.float16
+        need = K.prefill_attn_workspace_bytes(length, hq, hkv, start, fp16)
+        assert need > 0, "a split case"
+        ws = torch.full((need,), 0xFF, dtype=torch.uint8, device=gpu)  # NaN partials where nothing is written
+        args = (q.to(gpu), k.to(gpu), v.to(gpu), gate.to(gpu), kv.k[0], kv.v[0], kv.page_table[0])
+        stage = torch.empty(K.prefill_stage_bytes(length, hkv), dtype=torch.uint8, device=gpu) if staged else None
+        kw = dict(start=start, inv_freq=inv, scale=SCALE, stage=stage)
+        whole = K.attn_prefill(*args, **kw)
+        split = K.attn_prefill(*args, **kw, workspace=ws)
+        small = K.attn_prefill(*args, **kw, workspace=ws[:need - 16])  # too small: unsplit
+        assert torch.equal(whole, small)
+        vmax = float(max(v.abs().max(), v0.abs().max()))
+        tol = 4 * vmax * (2.0 ** -11 if fp16 else 2.0 ** -16) + 1e-5
+        assert float((split - whole).abs().max()) <= tol
