@@ -7,12 +7,20 @@
 // 0 .. start + t; the output is softmax(q K^T * scale) V * sigmoid(gate).
 //
 // Two launches: the prompt's k (rotated) and v go into the pages first (the
-// append kernel in sequence mode), then one workgroup per (16-token query
-// block, KV head) streams the keys 0 .. last query of the block in blocks of
-// 32 keys (two pages).
+// append kernel in sequence mode), then one workgroup per (query block of 16
+// or 32 tokens, KV head[, piece of its keys]) streams the keys 0 .. last query
+// of the block in blocks of 32 keys (two pages); a third launch merges the
+// pieces where query blocks are split.
+//   * bound by LDS operand reads and the softmax between the MFMAs: with 16
+//     tokens a wave reads one operand (8 cycles of the CU's LDS) per 16-cycle
+//     MFMA of its SIMD, so the MFMAs could run half the time at best (16384
+//     tokens: 2.25 ms, 0.98 PFLOP/s); with 32 tokens (fp16 operands: q 64 and
+//     O 128 of the 256 registers) each operand feeds two, 1.82 ms, 1.21
+//     PFLOP/s on the same box, where a large fp16 matrix product of the
+//     library reaches 1.5;
 //   * 8 waves, one query head each (GQA group <= 8), two waves per SIMD: one
 //     wave's softmax (VALU, transcendental) overlaps the other's MFMAs, and
-//     every key block fetched serves 16 tokens x 8 heads;
+//     every key block fetched serves the block's tokens x 8 heads;
 //   * key blocks travel HBM/L2 -> LDS by direct-to-LDS loads into a 4-slot
 //     ring, in pairs two blocks ahead of the one being computed, with no
 //     registers in flight and one barrier per pair;
@@ -86,13 +94,13 @@ struct PrefillAttnArgs {
 // rest.  Piece s exists for the query blocks qb >= first_query_block(s).  A
 // launch lists the pieces by s, each s from the last query block down, and
 // both kernels find a piece's index by the same counts.
-__host__ __device__ inline int first_query_block(int s, int chunk, int start, int nqb) {
+__host__ __device__ inline int first_query_block(int s, int chunk, int start, int nqb, int qt) {
   if (s == 0) return 0;
   const int64_t k0 = (int64_t)s * chunk * 32 - start;  // query tokens from here on see the piece's first key
-  return k0 <= 0 ? 0 : static_cast<int>(k0 + 15 < (int64_t)16 * nqb ? (k0 + 15) / 16 : nqb);
+  return k0 <= 0 ? 0 : static_cast<int>(k0 + qt - 1 < (int64_t)qt * nqb ? (k0 + qt - 1) / qt : nqb);
 }
-__host__ __device__ inline int query_block_pieces(int qb, int chunk, int start) {
-  return chunk ? 1 + (start + 16 * qb) / (32 * chunk) : 1;
+__host__ __device__ inline int query_block_pieces(int qb, int chunk, int start, int qt) {
+  return chunk ? 1 + (start + qt * qb) / (32 * chunk) : 1;
 }
 
 // Key held by row r (0..15) of score tile m (0, 1) of a 32-key block, as
@@ -110,6 +118,12 @@ __device__ __forceinline__ float max3_f(float a, float b, float c) {
   return r;
 }
 
+// acc + the two fp16 values of w (exact products with 1, fp32 sum)
+__device__ __forceinline__ float sum_pair_f16(uint32_t w, float acc) {
+  typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+  return __builtin_amdgcn_fdot2(__builtin_bit_cast(h2, w), h2{1, 1}, acc, false);
+}
+
 __device__ __forceinline__ float swap_max(float x, bool rows16) {
   const auto s = rows16 ? __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false)
                         : __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
@@ -122,22 +136,29 @@ __device__ __forceinline__ float swap_sum(float x, bool rows16) {
   return __uint_as_float(s[0]) + __uint_as_float(s[1]);
 }
 
-template <int AT, int KVT>
+template <int AT, int KVT, int NC>
 __global__ __launch_bounds__(kPrefillThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_prefill_kernel(
     PrefillAttnArgs a, const int32_t* __restrict__ pt) {
   using KV = Kv16<KVT>;
   // bf16 operands carry q and the probabilities as hi + lo pairs; fp16 ones
   // keep 11 significant bits in the hi part alone, which is enough here
   constexpr bool kSplit = KVT == RIA_DT_BF16;
-  const int nqb = (a.length + 15) / 16;
+  static_assert(NC == 1 || !kSplit, "two column tiles of hi + lo operands do not fit the registers");
+  constexpr int QT = 16 * NC;             // tokens of a query block
+  constexpr int KG = NC == 1 ? 8 : 1;     // 32-dim steps of K operands loaded at a time
+  constexpr int VG = NC == 1 ? 16 : 4;    // dim tiles of V^T operands loaded at a time
+  constexpr int NO = NC == 1 ? 17 : 16;   // O tiles of a column tile (17: the all-ones product)
+  const int nqb = (a.length + QT - 1) / QT;
   int piece = 0, unit = static_cast<int>(blockIdx.x);
   if (a.chunk)
-    for (int n; unit >= (n = (nqb - first_query_block(piece, a.chunk, a.start, nqb)) * a.num_kv_heads); unit -= n) ++piece;
+    for (int n; unit >= (n = (nqb - first_query_block(piece, a.chunk, a.start, nqb, QT)) * a.num_kv_heads); unit -= n) ++piece;
   const int qb = nqb - 1 - unit / a.num_kv_heads;  // heaviest blocks first
   const int kvh = unit % a.num_kv_heads;
-  const int pieces = query_block_pieces(qb, a.chunk, a.start);
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int n = lane & 15;   // MFMA column (token 16 qb + n) / row (key or dim)
+  const int pieces = query_block_pieces(qb, a.chunk, a.start, QT);
+  const int tid = threadIdx.x, lane = tid & 63;
+  // in a scalar register: the copies' LDS destinations and bases are then scalar
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n = lane & 15;   // MFMA column (token QT qb + 16 c + n) / row (key or dim)
   const int g4 = lane >> 4;  // lane group: k slice of the operands, row group of the results
 
   __shared__ __attribute__((aligned(16))) unsigned char smem[kPrefillLds];
@@ -146,15 +167,11 @@ __global__ __launch_bounds__(kPrefillThreads) __attribute__((amdgpu_waves_per_eu
 
   const bool head_ok = wave < a.group;
   const int head = kvh * a.group + wave;
-  const int t_row = 16 * qb + n;
-  const bool row_ok = head_ok && t_row < a.length;
-  const int qpos = a.start + t_row;
-  const int ctx_total = a.start + a.length;   // keys that exist
-  const int qlim = min(qpos, ctx_total - 1);  // last key this column sees
+  const int ctx_total = a.start + a.length;  // keys that exist
 
   // ---- q operands: column n, dims 32 kd + 8 g4 + j, RoPE'd, scaled by
   //      scale * log2(e) (scores come out in log2 units), as hi + lo pairs
-  u32x4 qh[8], ql[8];
+  u32x4 qh[NC][8], ql[8];
   // SEP: fp16 values converted one at a time, so hipcc folds the multiply
   // that produced each (q times its scale) into the conversion
   // (v_fma_mixlo_f16, one rounding); the probabilities, which no multiply
@@ -173,7 +190,11 @@ __global__ __launch_bounds__(kPrefillThreads) __attribute__((amdgpu_waves_per_eu
     lo = u32x4{l4[0], l4[1], l4[2], l4[3]};
   };
   const float sl2 = a.scale * 1.4426950408889634f;
-  {
+#pragma unroll
+  for (int c = 0; c < NC; ++c) {
+    const int t_row = QT * qb + 16 * c + n;
+    const bool row_ok = head_ok && t_row < a.length;
+    const int qpos = a.start + t_row;
     const int64_t base = (int64_t)t_row * a.q_stride + (int64_t)head * kAttnHeadDim + 8 * g4;
     auto load_q8 = [&](int kd, float (&y)[8]) {
       if (row_ok) {
@@ -219,7 +240,8 @@ __global__ __launch_bounds__(kPrefillThreads) __attribute__((amdgpu_waves_per_eu
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
         const float ang = mul_rn(pos, a.inv_freq[8 * g4 + j]);
-        const float cs = cosf(ang), sn = sinf(ang);
+        float cs, sn;
+        sincosf(ang, &sn, &cs);
         const float x1 = x[0][j], x2 = x[1][j];
         x[0][j] = add_rn(mul_rn(x1, cs), mul_rn(-x2, sn));
         x[1][j] = add_rn(mul_rn(x2, cs), mul_rn(x1, sn));
@@ -229,7 +251,7 @@ __global__ __launch_bounds__(kPrefillThreads) __attribute__((amdgpu_waves_per_eu
     for (int kd = 0; kd < 2; ++kd) {
 #pragma unroll
       for (int j = 0; j < 8; ++j) x[kd][j] *= sl2;
-      pack(x[kd], qh[kd], ql[kd], std::true_type{});
+      pack(x[kd], qh[c][kd], ql[kd], std::true_type{});
     }
 #pragma unroll
     for (int kd = 2; kd < 8; ++kd) {
@@ -237,16 +259,16 @@ __global__ __launch_bounds__(kPrefillThreads) __attribute__((amdgpu_waves_per_eu
       load_qn(kd, y);
 #pragma unroll
       for (int j = 0; j < 8; ++j) y[j] *= sl2;
-      pack(y, qh[kd], ql[kd], std::true_type{});
+      pack(y, qh[c][kd], ql[kd], std::true_type{});
     }
   }
 
-  const int q_last = a.start + min(16 * qb + 15, a.length - 1);  // last query position of the block
+  const int q_last = a.start + min(QT * qb + QT - 1, a.length - 1);  // last query position of the block
   const int npages = q_last / kPageTokens + 1;                   // <= pt_len (checked on the host)
   const int blk0 = piece * a.chunk;  // this piece's key blocks: blk0 (even) .. nblk - 1
   const int nblk = piece + 1 < pieces ? blk0 + a.chunk : (npages + 1) / 2;
   const int kmax = min(q_last, ctx_total - 1);  // last key any column of the block uses
-  const int q_first = a.start + 16 * qb;         // first query position of the block
+  const int q_first = a.start + QT * qb;         // first query position of the block
 
   // Direct-to-LDS copy of key block b (K and V tiles of pages 2b, 2b+1) into
   // ring slot b % 4: 4 loads of 16 bytes per thread; a page past the block's
@@ -254,37 +276,50 @@ __global__ __launch_bounds__(kPrefillThreads) __attribute__((amdgpu_waves_per_eu
   auto slot_of = [&](int b) { return ring + (b % kRingSlots) * kSlotVec; };
   auto issue = [&](int b) {
     u32x4* slot = slot_of(b);
+    int ln = lane;
+    asm volatile("" : "+v"(ln));  // its multiples computed here, not held over the loop
 #pragma unroll
     for (int pg = 0; pg < 2; ++pg) {
       const int p = 2 * b + pg;
       int phys = p < npages ? (a.staged ? p : pt[p]) : 0;
       phys = (phys < 0 || phys >= a.num_pages) ? 0 : phys;  // unallocated entries never fault
       const int64_t tile = (int64_t)phys * a.num_kv_heads + kvh;
-      const u32x4* kp = reinterpret_cast<const u32x4*>(a.k_cache + tile * kTile);
-      const u32x4* vp = reinterpret_cast<const u32x4*>(a.v_cache + tile * kTile);
+      // through a buffer resource per tile, in scalar registers, so the lane's
+      // part of the address is a 32-bit offset
+      const auto kr = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(a.k_cache + tile * kTile), 0, kTile * 2,
+                                                        kBufferWord3);
+      const auto vr = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(a.v_cache + tile * kTile), 0, kTile * 2,
+                                                        kBufferWord3);
       const int v = wave * 64;  // this wave's 64 vectors of each tile; lane l lands at +l
-      __builtin_amdgcn_global_load_lds(kp + v + lane, slot + pg * kSlotK1 + v, 16, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(kr, slot + pg * kSlotK1 + v, 16, 16 * ln, 16 * v, 0, 0);
       // V^T position (half, dim) = v + lane holds tile vector 2 dim + half
-      const int vdim = (wave & 3) * 64 + lane, vhalf = wave >> 2;
-      __builtin_amdgcn_global_load_lds(vp + 2 * vdim + vhalf, slot + kSlotV + pg * kTileVec + v, 16, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(vr, slot + kSlotV + pg * kTileVec + v, 16, 32 * ln,
+                                               32 * (wave & 3) * 64 + 16 * (wave >> 2), 0, 0);
     }
   };
 
-  // O^T tiles: dims 16 dt + 4 g4 + i, column n; o[16] is the product with an
-  // all-ones V^T tile, every row the sum of the column's probabilities as
-  // the MFMAs weighted V with them (the softmax's normaliser, no VALU adds
-  // and no cross-lane sum)
-  f32x4 o[17];
+  // O^T tiles: dims 16 dt + 4 g4 + i, column n.  The softmax's normaliser is
+  // the sum of the probabilities as the MFMAs weight V with them.  One column
+  // tile: o[16], the product with an all-ones V^T tile, every row that sum (no
+  // VALU adds and no cross-lane sum).  Two: l_run, the lane's own keys' part
+  // of it by v_dot2, summed across lanes at the end (the eight registers of
+  // the all-ones tiles are not there).
+  f32x4 o[NC][NO];
+  float m_run[NC], l_run[NC];
 #pragma unroll
-  for (int dt = 0; dt < 17; ++dt) o[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float m_run = -INFINITY;
+  for (int c = 0; c < NC; ++c) {
+#pragma unroll
+    for (int dt = 0; dt < NO; ++dt) o[c][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    m_run[c] = -INFINITY;
+    l_run[c] = 0.f;
+  }
   constexpr uint32_t kOne2 = KVT == RIA_DT_F16 ? 0x3C003C00u : 0x3F803F80u;  // two 16-bit 1.0
 
-  // K operand rows of this lane (row n of both score tiles): vector offset of
-  // token tile_row_token(m, n) of page tile_row_page(n); dims 32 kd + 8 g4 ..
-  // + 7 are dim group q8 = 4 kd + g4 at vector ((q8 % 8) * 4 + q8 / 8) * 16.
-  const int k_row0 = tile_row_page(n) * kSlotK1 + tile_row_token(0, n);
-  const int k_row1 = tile_row_page(n) * kSlotK1 + tile_row_token(1, n);
+  // K operands of this lane (row n of score tile m, dims 32 kd + 8 g4 .. + 7):
+  // token tile_row_token(m, n) of page tile_row_page(n), dim group q8 = 4 kd +
+  // g4 at vector ((q8 % 8) * 4 + q8 / 8) * 16, so k_vec + 256 (kd % 2) +
+  // 16 (kd / 2) + 4 m.
+  const int k_vec = tile_row_page(n) * kSlotK1 + tile_row_token(0, n) + 64 * g4;
   // V^T operand of this lane for dim tile dt: dim 16 dt + n, tokens
   // 8 (g4 % 2) .. + 7 of page g4 / 2 (one 16-byte vector).
   const int v_vec = kSlotV + (g4 >> 1) * kTileVec + (g4 & 1) * 256 + n;
@@ -296,95 +331,129 @@ __global__ __launch_bounds__(kPrefillThreads) __attribute__((amdgpu_waves_per_eu
   //
   // ---- scores of block b: two 16-key tiles; q_hi and q_lo products in separate
   //      accumulators so no MFMA waits on the one just before it
-  auto qk = [&](int b, f32x4 (&sc)[2]) {
+  auto qk = [&](int b, f32x4 (&sc)[NC][2]) {
     const u32x4* slot = slot_of(b);
-    u32x4 kop[8][2];
+    u32x4 kop[8 / KG > 1 ? 2 : 1][KG][2];
+    auto load_k = [&](int g, u32x4 (&dst)[KG][2]) {
 #pragma unroll
-    for (int kd = 0; kd < 8; ++kd) {
-      const int q8 = 4 * kd + g4;
-      const int goff = ((q8 & 7) * 4 + (q8 >> 3)) * kPageTokens;
-      kop[kd][0] = slot[k_row0 + goff];
-      kop[kd][1] = slot[k_row1 + goff];
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    f32x4 acc[4];
-#pragma unroll
-    for (int t = 0; t < 4; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int kd = 0; kd < 8; ++kd) {
-      acc[0] = KV::mfma_k32(kop[kd][0], qh[kd], acc[0]);
-      acc[1] = KV::mfma_k32(kop[kd][1], qh[kd], acc[1]);
-      if (kSplit) {
-        acc[2] = KV::mfma_k32(kop[kd][0], ql[kd], acc[2]);
-        acc[3] = KV::mfma_k32(kop[kd][1], ql[kd], acc[3]);
+      for (int i = 0; i < KG; ++i) {
+        const int kd = KG * g + i;
+        dst[i][0] = slot[k_vec + 256 * (kd & 1) + 16 * (kd >> 1)];
+        dst[i][1] = slot[k_vec + 256 * (kd & 1) + 16 * (kd >> 1) + 4];
       }
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    sc[0] = kSplit ? acc[0] + acc[2] : acc[0];
-    sc[1] = kSplit ? acc[1] + acc[3] : acc[1];
-  };
-
-  auto load_v = [&](int b, u32x4 (&vop)[17]) {
-    const u32x4* slot = slot_of(b);
+    };
+    load_k(0, kop[0]);
+    __builtin_amdgcn_sched_barrier(0);  // groups land in order
+    f32x4 acc[NC][2], acl[2];
 #pragma unroll
-    for (int dt = 0; dt < 16; ++dt) vop[dt] = slot[v_vec + 16 * dt];
-  };
-
-  // ---- online softmax of block b (log2 units), then O^T += V^T P^T over its 32 keys
-  auto softmax_pv = [&](int b, const f32x4 (&sc)[2]) {
-    u32x4 vop[17];
-    load_v(b, vop);
-    vop[16] = u32x4{kOne2, kOne2, kOne2, kOne2};
-    __builtin_amdgcn_sched_barrier(0);
-    float s[8];
+    for (int m = 0; m < 2; ++m) {
+      acl[m] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int c = 0; c < NC; ++c) acc[c][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+#pragma unroll
+    for (int g = 0; g < 8 / KG; ++g) {
+      if (g + 1 < 8 / KG) load_k(g + 1, kop[(g + 1) & 1]);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < KG; ++i)
+#pragma unroll
+        for (int m = 0; m < 2; ++m) {
+          const int kd = KG * g + i;
+#pragma unroll
+          for (int c = 0; c < NC; ++c) acc[c][m] = KV::mfma_k32(kop[g & 1][i][m], qh[c][kd], acc[c][m]);
+          if (kSplit) acl[m] = KV::mfma_k32(kop[g & 1][i][m], ql[kd], acl[m]);
+        }
+      __builtin_amdgcn_sched_barrier(0);
+    }
 #pragma unroll
     for (int m = 0; m < 2; ++m)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) s[4 * m + i] = sc[m][i];
-    if (32 * b + 31 > q_first) {
-      // blocks reaching past the block's first query need the causal mask
+      for (int c = 0; c < NC; ++c) sc[c][m] = kSplit ? acc[c][m] + acl[m] : acc[c][m];
+  };
+
+  // ---- online softmax of block b (log2 units), then O^T += V^T P^T over its 32 keys
+  auto softmax_pv = [&](int b, const f32x4 (&sc)[NC][2]) {
+    const u32x4* slot = slot_of(b);
+    u32x4 vop[16 / VG > 1 ? 2 : 1][VG];
+    auto load_v = [&](int g, u32x4 (&dst)[VG]) {
+#pragma unroll
+      for (int i = 0; i < VG; ++i) dst[i] = slot[v_vec + 16 * (VG * g + i)];
+    };
+    load_v(0, vop[0]);
+    __builtin_amdgcn_sched_barrier(0);
+    u32x4 ph[NC], pl;
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      float s[8];
 #pragma unroll
       for (int m = 0; m < 2; ++m)
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-          if (32 * b + 8 * g4 + 4 * m + i > qlim) s[4 * m + i] = -INFINITY;
+        for (int i = 0; i < 4; ++i) s[4 * m + i] = sc[c][m][i];
+      if (32 * b + 31 > q_first) {
+        // blocks reaching past the block's first query need the causal mask
+        int ln = lane;
+        asm volatile("" : "+v"(ln));  // computed here: held over the loop, these values cost registers
+        const int qlim = min(q_first + 16 * c + (ln & 15), ctx_total - 1);  // last key this column sees
+        const int key0 = 32 * b + 8 * (ln >> 4);
+#pragma unroll
+        for (int m = 0; m < 2; ++m)
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (key0 + 4 * m + i > qlim) s[4 * m + i] = -INFINITY;
+      }
+      // The probabilities against the running max go out at once; only a
+      // block with a score more than 2^8 above it (every column's first block
+      // among them) needs the column max (permlane swaps), the rescale and the
+      // probabilities again.  m_run is the same in the four lanes of a column,
+      // so a lane's own max decides as the column max would.
+      const float mloc = max3_f(max3_f(s[0], s[1], s[2]), max3_f(s[3], s[4], s[5]), max3_f(s[6], s[7], s[7]));
+      float pr[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        pr[j] = __builtin_amdgcn_exp2f(s[j] - m_run[c]);
+        asm volatile("" : "+v"(pr[j]));  // computed here, beside the vote, not sunk past the branch
+      }
+      if (__any(mloc > m_run[c] + 8.0f)) {
+        const float mx = swap_max(swap_max(mloc, true), false);
+        // m_run is finite from the first block on (the piece's first key is
+        // visible to every column), so masked scores give exp2(-inf) = 0
+        const bool grow = mx > m_run[c] + 8.0f;
+        const float m_new = grow ? mx : m_run[c];
+        const float alpha = __builtin_amdgcn_exp2f(m_run[c] - m_new);  // 0 on the first block, where o and l are 0
+#pragma unroll
+        for (int dt = 0; dt < NO; ++dt) o[c][dt] *= alpha;
+        l_run[c] *= alpha;
+        m_run[c] = m_new;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) pr[j] = __builtin_amdgcn_exp2f(s[j] - m_run[c]);
+      }
+      pack(pr, ph[c], pl, std::false_type{});
+      if constexpr (NC > 1) {
+        asm volatile("" : "+v"(ph[c]));  // packed here, before the next column tile's probabilities
+#pragma unroll
+        for (int j = 0; j < 4; ++j) l_run[c] = sum_pair_f16(ph[c][j], l_run[c]);
+      }
     }
-    // The probabilities against the running max go out at once; only a
-    // block with a score more than 2^8 above it (every column's first block
-    // among them) needs the column max (permlane swaps), the rescale and the
-    // probabilities again.  m_run is the same in the four lanes of a column,
-    // so a lane's own max decides as the column max would.
-    const float mloc = max3_f(max3_f(s[0], s[1], s[2]), max3_f(s[3], s[4], s[5]), max3_f(s[6], s[7], s[7]));
-    float pr[8];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      pr[j] = __builtin_amdgcn_exp2f(s[j] - m_run);
-      asm volatile("" : "+v"(pr[j]));  // computed here, beside the vote, not sunk past the branch
+    for (int g = 0; g < 16 / VG; ++g) {
+      if (g + 1 < 16 / VG) load_v(g + 1, vop[(g + 1) & 1]);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < VG; ++i)
+#pragma unroll
+        for (int c = 0; c < NC; ++c) o[c][VG * g + i] = KV::mfma_k32(vop[g & 1][i], ph[c], o[c][VG * g + i]);
+      if constexpr (NC == 1) {  // one group: all hi products, then all lo products (17 MFMAs between dependent ones)
+        const u32x4 ones{kOne2, kOne2, kOne2, kOne2};
+        o[0][16] = KV::mfma_k32(ones, ph[0], o[0][16]);
+        if (kSplit) {
+#pragma unroll
+          for (int dt = 0; dt < 16; ++dt) o[0][dt] = KV::mfma_k32(vop[0][dt], pl, o[0][dt]);
+          o[0][16] = KV::mfma_k32(ones, pl, o[0][16]);
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
     }
-    if (__any(mloc > m_run + 8.0f)) {
-      const float mx = swap_max(swap_max(mloc, true), false);
-      // m_run is finite from the first block on (the piece's first key is
-      // visible to every column), so masked scores give exp2(-inf) = 0
-      const bool grow = mx > m_run + 8.0f;
-      const float m_new = grow ? mx : m_run;
-      const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);  // 0 on the first block, where o and l are 0
-#pragma unroll
-      for (int dt = 0; dt < 17; ++dt) o[dt] *= alpha;
-      m_run = m_new;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) pr[j] = __builtin_amdgcn_exp2f(s[j] - m_run);
-    }
-    u32x4 ph, pl;
-    pack(pr, ph, pl, std::false_type{});
-    __builtin_amdgcn_sched_barrier(0);
-    // all hi products, then all lo products: 17 MFMAs between dependent ones
-#pragma unroll
-    for (int dt = 0; dt < 17; ++dt) o[dt] = KV::mfma_k32(vop[dt], ph, o[dt]);
-    if (kSplit) {
-#pragma unroll
-      for (int dt = 0; dt < 17; ++dt) o[dt] = KV::mfma_k32(vop[dt], pl, o[dt]);
-    }
-    __builtin_amdgcn_sched_barrier(0);
   };
 
   // Key blocks arrive in pairs, two blocks ahead.  At an even block every
@@ -397,7 +466,7 @@ __global__ __launch_bounds__(kPrefillThreads) __attribute__((amdgpu_waves_per_eu
   // all copies, not a count of them: it relies on no ordering among the
   // direct-to-LDS copies, only on each being written to LDS when the counter
   // no longer holds it; pairing gives each copy two iterations to land.
-  f32x4 sc[2];
+  f32x4 sc[NC][2];
   issue(blk0);
   if (blk0 + 1 < nblk) issue(blk0 + 1);
   for (int b = blk0; b < nblk; ++b) {
@@ -412,7 +481,8 @@ __global__ __launch_bounds__(kPrefillThreads) __attribute__((amdgpu_waves_per_eu
       // 0-probability keys cannot bring NaN/Inf from unwritten slots
 #pragma unroll
       for (int j2 = 0; j2 < 2; ++j2) {
-        const int vi = j2 * kPrefillThreads + tid;  // vector of the block's two V^T tiles
+        int vi = j2 * kPrefillThreads + tid;  // vector of the block's two V^T tiles
+        asm volatile("" : "+v"(vi));                 // computed here, not held over the loop
         const int m = vi / kTileVec;                 // page of the block
         const int half = (vi % kTileVec) >> 8;       // token half: tokens 8 half .. + 7 of one dim
         const int k0 = 32 * b + 16 * m + 8 * half;
@@ -429,43 +499,69 @@ __global__ __launch_bounds__(kPrefillThreads) __attribute__((amdgpu_waves_per_eu
       lds_barrier();
     }
 
+    // The scores' MFMAs go ahead of the other wave's softmax on this SIMD: the
+    // sooner a wave reaches its own softmax, the more of it runs beside MFMAs
+    // (hi + lo operands: 197 -> 185 us for 500 tokens after 12000).
+    __builtin_amdgcn_s_setprio(1);
     qk(b, sc);
+    __builtin_amdgcn_s_setprio(0);
     softmax_pv(b, sc);
   }
 
+  if (NC > 1) {
+#pragma unroll
+    for (int c = 0; c < NC; ++c) l_run[c] = swap_sum(swap_sum(l_run[c], true), false);
+  } else {
+    l_run[0] = o[0][NO - 1][0];
+  }
   if (pieces > 1) {  // a split query block: the combine launch merges the pieces
     if (!head_ok) return;
-    const int64_t row = ((int64_t)blockIdx.x * a.group + wave) * 16 + n;
-    float* pp = a.part + row * kAttnHeadDim + 4 * g4;
 #pragma unroll
-    for (int dt = 0; dt < 16; ++dt) *reinterpret_cast<f32x4*>(pp + 16 * dt) = o[dt];
-    if (g4 == 0) a.part_ml[row] = float2{m_run, o[16][0]};
+    for (int c = 0; c < NC; ++c) {
+      const int64_t row = ((int64_t)blockIdx.x * a.group + wave) * QT + 16 * c + n;
+      float* pp = a.part + row * kAttnHeadDim + 4 * g4;
+#pragma unroll
+      for (int dt = 0; dt < 16; ++dt) *reinterpret_cast<f32x4*>(pp + 16 * dt) = o[c][dt];
+      if (g4 == 0) a.part_ml[row] = float2{m_run[c], l_run[c]};
+    }
     return;
   }
   // ---- normalise, stage (the ring is dead once every wave has left the loop), gate, store
   lds_barrier();
-  const float l_tot = o[16][0];
-  const float inv = 1.0f / l_tot;  // every valid query sees at least itself
-  float* st = stage + (wave * 16 + n) * kStagePitch;
 #pragma unroll
-  for (int dt = 0; dt < 16; ++dt)
-    *reinterpret_cast<f32x4*>(st + 16 * dt + 4 * g4) = o[dt] * inv;
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-  if (!head_ok) return;
-  for (int r = 0; r < 16; ++r) {
-    const int t = 16 * qb + r;
-    if (t >= a.length) break;
+  for (int c = 0; c < NC; ++c) {
+    const float inv = 1.0f / l_run[c];  // every valid query sees at least itself
+    float* st = stage + (wave * 16 + n) * kStagePitch;
+#pragma unroll
+    for (int dt = 0; dt < 16; ++dt) *reinterpret_cast<f32x4*>(st + 16 * dt + 4 * g4) = o[c][dt] * inv;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    if (!head_ok) return;
+    // Gate rows in batches of 8 loads (rows past the prompt repeat its last
+    // one): row by row, each row's load latency was exposed, 16 in a row.
     const int d = 4 * lane;
-    // one 16-byte read of the staged row (element reads would hit 4-way bank conflicts)
-    const f32x4 row = *reinterpret_cast<const f32x4*>(stage + (wave * 16 + r) * kStagePitch + d);
-    float g[4], y[4];
-    load_act4<AT>(a.gate, (int64_t)t * a.gate_stride + (int64_t)head * kAttnHeadDim + d, g);
+    const int t0 = QT * qb + 16 * c;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      y[i] = AT == RIA_DT_BF16 ? gate_mul_to_bf16(row[i], g[i]) : mul_rn(row[i], sigmoid_f(g[i]));
-    store_act4<AT>(a.out, ((int64_t)t * a.num_q_heads + head) * kAttnHeadDim + d, y);
+    for (int r0 = 0; r0 < 16; r0 += 8) {
+      float g[8][4];
+#pragma unroll
+      for (int r = 0; r < 8; ++r)
+        load_act4<AT>(a.gate, (int64_t)min(t0 + r0 + r, a.length - 1) * a.gate_stride + (int64_t)head * kAttnHeadDim + d, g[r]);
+#pragma unroll
+      for (int r = 0; r < 8; ++r) {
+        const int t = t0 + r0 + r;
+        if (t >= a.length) break;
+        // one 16-byte read of the staged row (element reads would hit 4-way bank conflicts)
+        const f32x4 row = *reinterpret_cast<const f32x4*>(stage + (wave * 16 + r0 + r) * kStagePitch + d);
+        float y[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          y[i] = AT == RIA_DT_BF16 ? gate_mul_to_bf16(row[i], g[r][i]) : mul_rn(row[i], sigmoid_f(g[r][i]));
+        store_act4<AT>(a.out, ((int64_t)t * a.num_q_heads + head) * kAttnHeadDim + d, y);
+      }
+    }
+    __builtin_amdgcn_wave_barrier();  // the next tile's rows take the same region after these reads
   }
 }
 
@@ -474,14 +570,14 @@ __global__ __launch_bounds__(kPrefillThreads) __attribute__((amdgpu_waves_per_eu
 // w_s = 2^(m_s - max m).  Bound by the partials' bytes (16 tokens x 8 heads x
 // 1 KB per piece, written and read once).
 template <int AT>
-__global__ __launch_bounds__(256) void attn_prefill_combine_kernel(PrefillAttnArgs a) {
+__global__ __launch_bounds__(256) void attn_prefill_combine_kernel(PrefillAttnArgs a, int qt) {
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int64_t r = (int64_t)blockIdx.x * 4 + wave;
   const int t = static_cast<int>(r / a.num_q_heads), head = static_cast<int>(r % a.num_q_heads);
   if (t >= a.length) return;
-  const int nqb = (a.length + 15) / 16, qb = t / 16;
-  const int pieces = query_block_pieces(qb, a.chunk, a.start);
+  const int nqb = (a.length + qt - 1) / qt, qb = t / qt;
+  const int pieces = query_block_pieces(qb, a.chunk, a.start, qt);
   if (pieces == 1) return;  // its workgroup stored the result
   const int d = 4 * lane;
   float g[4], y[4];
@@ -489,7 +585,7 @@ __global__ __launch_bounds__(256) void attn_prefill_combine_kernel(PrefillAttnAr
   const int kvh = head / a.group;
   // row of piece s in the partials: its index in the launch, this head and token
   auto row_of = [&](int s, int64_t before) {
-    return ((before + (int64_t)(nqb - 1 - qb) * a.num_kv_heads + kvh) * a.group + head % a.group) * 16 + t % 16;
+    return ((before + (int64_t)(nqb - 1 - qb) * a.num_kv_heads + kvh) * a.group + head % a.group) * qt + t % qt;
   };
   int64_t before = 0;
   float m = -INFINITY, l = 0.f;
@@ -503,7 +599,7 @@ __global__ __launch_bounds__(256) void attn_prefill_combine_kernel(PrefillAttnAr
       const int64_t row = row_of(s, before);
       ml[j] = a.part_ml[row];
       po[j] = *reinterpret_cast<const f32x4*>(a.part + row * kAttnHeadDim + d);
-      if (s0 + j + 1 < pieces) before += (int64_t)(nqb - first_query_block(s, a.chunk, a.start, nqb)) * a.num_kv_heads;
+      if (s0 + j + 1 < pieces) before += (int64_t)(nqb - first_query_block(s, a.chunk, a.start, nqb, qt)) * a.num_kv_heads;
     }
     float mx = m;
 #pragma unroll
@@ -530,60 +626,75 @@ __global__ __launch_bounds__(256) void attn_prefill_combine_kernel(PrefillAttnAr
 }
 
 template <int AT>
-static void launch_prefill(const PrefillAttnArgs& a, const int32_t* pt, int kv_dtype, dim3 grid, hipStream_t st) {
-  if (kv_dtype == RIA_DT_F16)
-    hipLaunchKernelGGL((attn_prefill_kernel<AT, RIA_DT_F16>), grid, dim3(kPrefillThreads), 0, st, a, pt);
+static void launch_prefill(const PrefillAttnArgs& a, const int32_t* pt, int kv_dtype, int qt, dim3 grid, hipStream_t st) {
+  if (kv_dtype == RIA_DT_BF16)
+    hipLaunchKernelGGL((attn_prefill_kernel<AT, RIA_DT_BF16, 1>), grid, dim3(kPrefillThreads), 0, st, a, pt);
+  else if (qt == 16)
+    hipLaunchKernelGGL((attn_prefill_kernel<AT, RIA_DT_F16, 1>), grid, dim3(kPrefillThreads), 0, st, a, pt);
   else
-    hipLaunchKernelGGL((attn_prefill_kernel<AT, RIA_DT_BF16>), grid, dim3(kPrefillThreads), 0, st, a, pt);
+    hipLaunchKernelGGL((attn_prefill_kernel<AT, RIA_DT_F16, 2>), grid, dim3(kPrefillThreads), 0, st, a, pt);
   if (a.chunk) {
     const int64_t rows = (int64_t)a.length * a.num_q_heads;
-    hipLaunchKernelGGL((attn_prefill_combine_kernel<AT>), dim3(static_cast<unsigned>((rows + 3) / 4)), dim3(256), 0, st, a);
+    hipLaunchKernelGGL((attn_prefill_combine_kernel<AT>), dim3(static_cast<unsigned>((rows + 3) / 4)), dim3(256), 0, st, a, qt);
   }
 }
 
-// How a prompt's query blocks are split (PrefillAttnArgs::chunk) and the
-// pieces that makes.  One workgroup per CU runs at a time, so the launch
-// takes about max(longest piece, work / CUs): a prompt whose query blocks
-// number fewer than the CUs, or whose last blocks hold most keys, is cut into
-// pieces until the cut costs more (the prologue of each piece, the partials'
-// traffic, the combine launch) than it evens out.  Costs in key blocks of the
-// fp16 kernel (about 1 us each), from kernel times on MI355X: prologue and
-// epilogue of a whole query block 16, of a piece 9; a bf16 block (hi + lo
-// operands) 1.5; combine 6 + one per 15 pieces.
+// How a prompt's query blocks are formed (16 or 32 tokens) and split
+// (PrefillAttnArgs::chunk).  One workgroup per CU runs at a time, so a launch
+// takes about max(longest piece, work / CUs).  Blocks of 32 tokens do twice
+// the MFMAs per LDS operand read and win once every CU is busy (8000 tokens
+// 604 -> 471 us), but halve the workgroups and double the longest chain (4096
+// tokens: 179 us in blocks of 16, 206 in blocks of 32).  A prompt whose query
+// blocks number fewer than the CUs, or whose last blocks hold most keys, is
+// cut into pieces where the prologue of each piece, the partials' traffic and
+// the combine launch cost less than it evens out (500 tokens after 12000: 585
+// -> 190 us; 1000 tokens 49 -> 43; 300 tokens 26.2 whole, 27.2 cut).
+// Costs in microseconds on MI355X, from a sweep of both choices over 17 ..
+// 8000 tokens after 0 .. 12000: a 32-key block (while other CUs idle, while
+// all are busy) of 16 tokens with fp16 keys 1.05, 1.15, of 32 tokens 1.36,
+// 1.65, of 16 tokens with bf16 hi + lo operands 1.8; prologue and epilogue 14
+// per 16 tokens; combine 6 + one per 40 pieces of 16 tokens.
 struct PrefillPlan {
+  int qt;          // tokens of a query block
   int chunk;       // 0: unsplit
   int64_t pieces;  // workgroups of the launch
 };
-static PrefillPlan plan_prefill(int length, int start, int num_kv_heads, bool fp16_keys) {
-  const int cus = device_cus(), nqb = (length + 15) / 16;
+static PrefillPlan plan_prefill(int length, int start, int num_kv_heads, bool fp16_keys, int max_pieces) {
+  const int cus = device_cus();
   const int most = ((start + length - 1) / kPageTokens + 2) / 2;  // key blocks of the last query block
-  const double per_block = fp16_keys ? 1.0 : 1.5;
-  PrefillPlan best{0, (int64_t)nqb * num_kv_heads};
+  PrefillPlan best{};
   double best_cost = -1;
-  for (int k = 1; k <= kMaxPieces; ++k) {
-    const int chunk = k == 1 ? 0 : ((most + k - 1) / k + 1) / 2 * 2;
-    if (k > 1 && chunk < kMinPieceBlocks) break;
-    int64_t pieces = 0;
-    for (int s = 0; s < k; ++s) pieces += (int64_t)(nqb - first_query_block(s, chunk, start, nqb)) * num_kv_heads;
-    // key blocks in all: query block qb has (start + 16 qb) / 32 + 1 of them
-    const double work = (double)num_kv_heads * nqb * ((start + 8.0 * nqb) / 32 + 1) * per_block + pieces * (k == 1 ? 16.0 : 9.0);
-    const double longest = (k == 1 ? most : chunk + 1) * per_block + (k == 1 ? 16.0 : 9.0);
-    double cost = std::max(longest, work / cus);
-    if (k > 1) {  // whole query blocks run longest first and end together; pieces of several sizes do not
-      if (pieces > 2 * cus) continue;
-      if (pieces > cus) cost = std::max(cost, work / cus + longest / 2);
-      cost += 6.0 + pieces / 15.0;
-    }
-    if (best_cost < 0 || cost < best_cost) {
-      best_cost = cost;
-      best = PrefillPlan{chunk, pieces};
+  for (int qt = 16; qt <= (fp16_keys ? 32 : 16); qt += 16) {
+    const int nqb = (length + qt - 1) / qt;
+    const double block = !fp16_keys ? 1.8 : qt == 16 ? 1.05 : 1.36;
+    const double block_busy = !fp16_keys ? 1.8 : qt == 16 ? 1.15 : 1.65;
+    const double fixed = 14.0 * qt / 16;
+    for (int k = 1; k <= max_pieces; ++k) {
+      const int chunk = k == 1 ? 0 : ((most + k - 1) / k + 1) / 2 * 2;
+      if (k > 1 && chunk < kMinPieceBlocks) break;
+      int64_t pieces = 0;
+      for (int s = 0; s < k; ++s) pieces += (int64_t)(nqb - first_query_block(s, chunk, start, nqb, qt)) * num_kv_heads;
+      if (k > 1 && pieces * qt > 32 * cus) continue;  // partials of at most 64 MB for 8 heads a group
+      // key blocks in all: query block qb has about (start + qt qb) / 32 + 1 of them
+      const double work =
+          (double)num_kv_heads * nqb * ((start + 0.5 * qt * nqb) / 32 + 1) * block_busy + pieces * fixed;
+      const double longest = (k == 1 ? most : chunk + 1) * block + fixed;
+      double cost = std::max(longest, work / cus);
+      if (k > 1) {  // whole query blocks run longest first and end together; pieces of several sizes do not
+        if (pieces > cus) cost = std::max(cost, work / cus + longest / 4);
+        cost += 6.0 + pieces * qt / 640.0;
+      }
+      if (best_cost < 0 || cost < best_cost) {
+        best_cost = cost;
+        best = PrefillPlan{qt, chunk, pieces};
+      }
     }
   }
   return best;
 }
 
 static int64_t partial_bytes(const PrefillPlan& p, int group) {
-  return p.chunk ? p.pieces * group * 16 * (int64_t)(kAttnHeadDim * sizeof(float) + sizeof(float2)) : 0;
+  return p.chunk ? p.pieces * group * p.qt * (int64_t)(kAttnHeadDim * sizeof(float) + sizeof(float2)) : 0;
 }
 
 }  // namespace ria
@@ -686,25 +797,24 @@ static int prefill_impl(int length, int num_q_heads, int num_kv_heads, const voi
     a.staged = 1;
     key_dtype = RIA_DT_F16;
   }
-  dim3 grid(static_cast<unsigned>(blocks));
+  PrefillPlan plan = plan_prefill(length, start_pos, num_kv_heads, key_dtype == RIA_DT_F16, workspace ? kMaxPieces : 1);
   if (workspace) {
     if (reinterpret_cast<uintptr_t>(workspace) % 16)
       return set_error(RIA_ERR_INVALID, "ria_attn_prefill: workspace must be 16-byte aligned");
-    const PrefillPlan plan = plan_prefill(length, start_pos, num_kv_heads, key_dtype == RIA_DT_F16);
-    if (plan.chunk && partial_bytes(plan, group) <= workspace_bytes) {  // a smaller workspace: no split
-      a.chunk = plan.chunk;
-      a.part = static_cast<float*>(workspace);
-      a.part_ml = reinterpret_cast<float2*>(a.part + plan.pieces * group * 16 * kAttnHeadDim);
-      grid.x = static_cast<unsigned>(plan.pieces);
-    }
+    if (partial_bytes(plan, group) > workspace_bytes)  // too small: no split
+      plan = plan_prefill(length, start_pos, num_kv_heads, key_dtype == RIA_DT_F16, 1);
+    a.chunk = plan.chunk;
+    a.part = static_cast<float*>(workspace);
+    a.part_ml = reinterpret_cast<float2*>(a.part + plan.pieces * group * plan.qt * kAttnHeadDim);
   }
+  const dim3 grid(static_cast<unsigned>(plan.pieces));
   hipStream_t st = static_cast<hipStream_t>(stream);
   if (act_dtype == RIA_DT_BF16)
-    launch_prefill<RIA_DT_BF16>(a, page_table_row, key_dtype, grid, st);
+    launch_prefill<RIA_DT_BF16>(a, page_table_row, key_dtype, plan.qt, grid, st);
   else if (act_dtype == RIA_DT_F16)
-    launch_prefill<RIA_DT_F16>(a, page_table_row, key_dtype, grid, st);
+    launch_prefill<RIA_DT_F16>(a, page_table_row, key_dtype, plan.qt, grid, st);
   else
-    launch_prefill<RIA_DT_F32>(a, page_table_row, key_dtype, grid, st);
+    launch_prefill<RIA_DT_F32>(a, page_table_row, key_dtype, plan.qt, grid, st);
   return check_launch("ria_attn_prefill");
 }
 }  // namespace ria
@@ -746,7 +856,7 @@ extern "C" int ria_attn_prefill_staged(int length, int num_q_heads, int num_kv_h
 extern "C" int64_t ria_attn_prefill_workspace_bytes(int length, int num_q_heads, int num_kv_heads, int32_t start_pos,
                                                     int fp16_keys) {
   if (length <= 0 || start_pos < 0 || num_kv_heads <= 0 || num_q_heads <= 0 || num_q_heads % num_kv_heads) return 0;
-  return partial_bytes(plan_prefill(length, start_pos, num_kv_heads, fp16_keys != 0), num_q_heads / num_kv_heads);
+  return partial_bytes(plan_prefill(length, start_pos, num_kv_heads, fp16_keys != 0, kMaxPieces), num_q_heads / num_kv_heads);
 }
 
 extern "C" int ria_attn_prefill_split(int length, int num_q_heads, int num_kv_heads, const void* q,

@@ -214,8 +214,8 @@ def test_attn_prefill_keeps_its_tolerance_margin(gpu, staged, bound):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("length,start,hq,hkv", [(1, 300, 16, 2), (17, 2047, 16, 2), (100, 1000, 6, 2),
-                                                  (333, 0, 16, 2), (500, 2100, 16, 2), (1000, 0, 16, 2), (130, 513, 4, 4)])
+@pytest.mark.parametrize("length,start,hq,hkv", [(1, 1300, 16, 2), (17, 2047, 16, 2), (100, 1000, 6, 2),
+                                                  (517, 0, 16, 2), (500, 7900, 16, 2), (1000, 0, 16, 2), (130, 813, 4, 4)])
 def test_attn_prefill_split_keys(gpu, length, start, hq, hkv):
     """Query blocks whose keys are split between workgroups against the unsplit
     launch, fp32 activations.  Both round the probabilities (fp16: 2^-11,
@@ -243,3 +243,28 @@ def test_attn_prefill_split_keys(gpu, length, start, hq, hkv):
         vmax = float(max(v.abs().max(), v0.abs().max()))
         tol = 4 * vmax * (2.0 ** -11 if fp16 else 2.0 ** -16) + 1e-5
         assert float((split - whole).abs().max()) <= tol
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("length,hq,hkv", [(6017, 16, 2), (6031, 16, 2), (6048, 6, 2)])
+@pytest.mark.parametrize("staged", [False, True], ids=["fp16 pages", "stage"])
+def test_attn_prefill_32_token_blocks(gpu, length, hq, hkv, staged):
+    """Long fp16-key prompts run in query blocks of 32 tokens.  Their first and
+    last tokens (remainders of 1, 15 and 32) against the same tokens in blocks
+    of 16: a short prompt of the first ones, and the last ones continued over
+    the prompt's own pages.  Same bound as the split launches; the stage's fp16
+    keys are compared on pages that hold the same fp16 values."""
+    announce(f"attn_prefill 32-token blocks: L={length}, Hq={hq}, {'stage' if staged else 'fp16 pages'}")
+    q, k, v, gate = (x.to(gpu) for x in _inputs(9 + length, length, hq, hkv, torch.float32))
+    inv = rope_inv_freq(10_000_000.0, 64).to(gpu)
+    kv = _cache(gpu, length, hkv, torch.float16)
+    stage = torch.empty(K.prefill_stage_bytes(length, hkv), dtype=torch.uint8, device=gpu) if staged else None
+    kw = dict(inv_freq=inv, scale=SCALE)
+    out = K.attn_prefill(q, k, v, gate, kv.k[0], kv.v[0], kv.page_table[0], start=0, stage=stage, **kw)
+    tol = 4 * float(v.abs().max()) * 2.0 ** -11 + 1e-5
+    n = 70
+    t0 = length - n
+    last = K.attn_prefill(q[t0:], k[t0:], v[t0:], gate[t0:], kv.k[0], kv.v[0], kv.page_table[0], start=t0, **kw)
+    first = K.attn_prefill(q[:n], k[:n], v[:n], gate[:n], kv.k[0], kv.v[0], kv.page_table[0], start=0, **kw)
+    assert float((out[t0:] - last).abs().max()) <= tol
+    assert float((out[:n] - first).abs().max()) <= tol
