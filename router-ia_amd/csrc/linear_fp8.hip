@@ -30,6 +30,9 @@
 //                        operands loaded row-contiguous into registers and
 //                        turned into MFMA operands through each wave's own
 //                        LDS region.
+//   linear_fp8_mm_kernel prompts (a few hundred rows and more): tiles of 256 x
+//                        256 or 128 x 128 over the whole K, both operands
+//                        converted once into a double buffer in LDS.
 #include <algorithm>
 #include <type_traits>
 #include <utility>
@@ -113,6 +116,7 @@ struct LinearArgs {
   int64_t x_stride;
   int m, k, count;
   int mt;               // rows of x per workgroup (streaming kernel): 64 or 128
+  int tiles;            // feature tiles of the group (many-row kernel)
   const float* norm_w;  // fused input RMSNorm (one-pass kernel, up to 4 rows of fp32 x), or null
   float norm_eps;
   int norm_dtype;       // the normed rows are rounded to this dtype, then to fp16
@@ -592,15 +596,10 @@ constexpr int kKsChunk = 64;
 // Eight bf16 values as eight fp16 values (round to nearest even: exact
 // within fp16's normal range), as F.linear's x.to(float16) gives them.
 __device__ __forceinline__ u32x4 bf16x8_to_f16x8(u32x4 v) {
-  typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+  using B16 = Kv16<RIA_DT_BF16>;
   u32x4 r;
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    h2 p;
-    p[0] = static_cast<_Float16>(__uint_as_float(v[j] << 16));
-    p[1] = static_cast<_Float16>(__uint_as_float(v[j] & 0xffff0000u));
-    r[j] = __builtin_bit_cast(uint32_t, p);
-  }
+  for (int j = 0; j < 4; ++j) r[j] = Kv16<RIA_DT_F16>::pack2(B16::lo_f32(v[j]), B16::hi_f32(v[j]));
   return r;
 }
 
@@ -847,6 +846,247 @@ __global__ __launch_bounds__(64 * NW) void linear_fp8_ks_kernel(const LinearArgs
   }
 }
 
+// Many rows (prompts): tiles of BM rows x BN features over the whole of K, 64
+// K a step, two wave groups.  Per step the workgroup's threads load x (fp16,
+// or bf16: XB) and fp8 weights row-contiguously into registers, convert them
+// once (weights to fp16(w8 s), the same values as every kernel here) and write
+// them to one half of a double buffer in LDS in MFMA operand order, while the
+// MFMAs read the other half; one barrier a step.  A tile of 256 x 256
+// dequantises a weight once per 256 rows (the K-split kernel once per 64, which
+// made it VALU-bound: 25 M weights x 256 row blocks at 16384 rows) and each
+// wave's 64 x 128 of results takes 24 operand reads for 64 MFMAs.  The two
+// waves of a SIMD are in different groups: the first converts the next step's
+// tile before its MFMAs, the second after, and the MFMAs have the higher wave
+// priority, so one's conversion (VALU) runs beside the other's MFMAs (both
+// after: 791 us for 16384 rows of 12352 features; no priority: 871).
+// 16384 rows x 12352 x 2048: 1638 -> 740 us, 1.12 PFLOP/s; the library's fp16
+// product of that shape takes 731.  The matrix cores are busy 56% of the
+// cycles, at a clock that falls as they get busier (1.7 GHz of 2.4).
+//
+// Every result is one accumulator over K in order, whatever the tile, and the
+// rows and K alone choose the kernel, so grouped and separate calls agree bit
+// for bit.
+//
+// LDS half: x, then weights, as 16-byte entries (8 K of one row): entry
+// (row tile rt, K piece q = 0 .. 7, row r) at (rt * 8 + q) * 16 + (r ^ swz(q)),
+// swz(q) = q for x and q & 6 for weights.  A store's 8 lanes (one row x 8
+// pieces of x; 2 rows x 4 alternate pieces of weights) hit 8 entries distinct
+// modulo 8.  An operand read takes lanes 0-3, 12-15 of one piece with lanes
+// 4-11 of the next in one pass, so two such pieces' XORs may differ in bits 0
+// and 1 only (bits 2 and 3 together): with x's q ^ 8 (q & 1) the kernel ran
+// 871 us against 758, 544 conflict cycles a step.
+template <int BM, int BN, int WM, int WN, bool XB>
+__global__ __launch_bounds__(64 * (BM / WM) * (BN / WN)) void linear_fp8_mm_kernel(const LinearArgs a) {
+  using F16 = Kv16<RIA_DT_F16>;
+  constexpr int NW = (BM / WM) * (BN / WN), NT = 64 * NW;
+  constexpr int MT = WM / 16, FT = WN / 16;      // row and feature tiles of a wave
+  constexpr int XL = BM * 8 / NT, WL = BN * 4 / NT;  // 16-byte loads of a thread per step
+  constexpr int kWRows = NT / 4;                 // weight rows of one load of the workgroup
+  static_assert(BM * 8 % NT == 0 && BN * 4 % NT == 0 && kFp8Block % kWRows == 0 && BN % kFp8Block == 0, "whole loads");
+  constexpr int kHalf = (BM + BN) * 8;           // 16-byte entries of one half
+  __shared__ u32x4 mm_lds[2 * kHalf];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n16 = lane & 15, g4 = lane >> 4;
+  // Workgroup ids congruent mod 8 share an XCD: each XCD takes a contiguous
+  // run of tiles in an order of 4 row blocks x every feature block, so its L2
+  // holds the rows of x it is working on while the weights stream past.
+  const int per_xcd = gridDim.x / 8;
+  const int order = static_cast<int>(blockIdx.x % 8) * per_xcd + static_cast<int>(blockIdx.x / 8);
+  const int mblocks = (a.m + BM - 1) / BM;
+  if (order >= mblocks * a.tiles) return;
+  const int g0 = order / (4 * a.tiles) * 4, gsz = min(4, mblocks - g0), in_g = order - g0 * a.tiles;
+  const int m0 = (g0 + in_g % gsz) * BM;
+  const int bx = in_g / gsz;
+  const uint8_t* w = a.p[0].w;
+  const float* scale = a.p[0].scale;
+  void* y = a.p[0].y;
+  int64_t y_stride = a.p[0].y_stride;
+  int n = a.p[0].n, y_dtype = a.p[0].y_dtype, y_add = a.p[0].y_add, tile0 = 0;
+#pragma unroll
+  for (int j = 1; j < kLinGroup; ++j)
+    if (j < a.count && bx >= a.p[j].tile0) {
+      w = a.p[j].w;
+      scale = a.p[j].scale;
+      y = a.p[j].y;
+      y_stride = a.p[j].y_stride;
+      n = a.p[j].n;
+      y_dtype = a.p[j].y_dtype;
+      y_add = a.p[j].y_add;
+      tile0 = a.p[j].tile0;
+    }
+  const int n0 = (bx - tile0) * BN;
+  const int steps = a.k / kKsChunk;
+  const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<void*>(a.x), 0, static_cast<int>(static_cast<uint32_t>(((int64_t)(a.m - 1) * a.x_stride + a.k) * 2)), kBufferWord3);
+  const __amdgpu_buffer_rsrc_t wr =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(w), 0, static_cast<int>(static_cast<uint32_t>((int64_t)n * a.k)), kBufferWord3);
+  // rows past the last token and features past n repeat the last one: computed, never stored
+  uint32_t xo[XL], wo[WL];
+  const float* sp[WL];  // the scale row of the features of load i (one block of 128)
+#pragma unroll
+  for (int i = 0; i < XL; ++i) {
+    const int u = tid + NT * i;
+    xo[i] = static_cast<uint32_t>((min(m0 + (u >> 3), a.m - 1) * a.x_stride + 8 * (u & 7)) * 2);
+  }
+#pragma unroll
+  for (int i = 0; i < WL; ++i) {
+    wo[i] = static_cast<uint32_t>(min(n0 + kWRows * i + (tid >> 2), n - 1) * a.k + 16 * (tid & 3));
+    sp[i] = scale + (int64_t)(min(n0 + kWRows * i, n - 1) / kFp8Block) * (a.k / kFp8Block);
+  }
+  // LDS entries: this thread's stores, this lane's operand reads
+  auto swz_x = [](int q) { return q; };
+  auto swz_w = [](int q) { return (q >> 1) << 1; };
+  const int x_st = ((tid >> 7) * 8 + (tid & 7)) * 16 + (((tid >> 3) & 15) ^ swz_x(tid & 7));  // load i: + 8 NT / 8 i rows
+  const int w_st = BM * 8 + ((tid >> 6) * 8 + 2 * (tid & 3)) * 16 + (((tid >> 2) & 15) ^ swz_w(2 * (tid & 3)));
+  const int wm = wave % (BM / WM), wn = wave / (BM / WM);
+  int x_rd[2], w_rd[2];
+#pragma unroll
+  for (int s = 0; s < 2; ++s) {
+    const int q = 4 * s + g4;
+    x_rd[s] = (wm * MT * 8 + q) * 16 + (n16 ^ swz_x(q));
+    w_rd[s] = BM * 8 + (wn * FT * 8 + q) * 16 + (n16 ^ swz_w(q));
+  }
+  u32x4 xs[XL], ws[WL];
+  float sc[WL];
+  auto load = [&](int c) __attribute__((always_inline)) {  // step c into registers (past the last: the last again)
+    const int ko = min(c, steps - 1) * kKsChunk;
+#pragma unroll
+    for (int i = 0; i < XL; ++i)
+      xs[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(xr, xo[i], 2 * ko, 0));
+#pragma unroll
+    for (int i = 0; i < WL; ++i) {
+      ws[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(wr, wo[i], ko, 0));
+      sc[i] = sp[i][ko / kFp8Block];
+    }
+  };
+  auto store = [&](int half) __attribute__((always_inline)) {  // the loaded step, converted, into an LDS half
+    u32x4* d = mm_lds + half * kHalf;
+#pragma unroll
+    for (int i = 0; i < WL; ++i) {
+      const u32x4 v = ws[i];
+      const float s = sc[i];
+      d[w_st + kWRows * 8 * i] = u32x4{dequant_pair<false>(v[0], s), dequant_pair<true>(v[0], s),
+                                       dequant_pair<false>(v[1], s), dequant_pair<true>(v[1], s)};
+      d[w_st + kWRows * 8 * i + 16] = u32x4{dequant_pair<false>(v[2], s), dequant_pair<true>(v[2], s),
+                                            dequant_pair<false>(v[3], s), dequant_pair<true>(v[3], s)};
+    }
+#pragma unroll
+    for (int i = 0; i < XL; ++i) d[x_st + NT * i] = XB ? bf16x8_to_f16x8(xs[i]) : xs[i];
+  };
+  f32x4 acc[FT][MT];
+#pragma unroll
+  for (int f = 0; f < FT; ++f)
+#pragma unroll
+    for (int r = 0; r < MT; ++r) acc[f][r] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // Products of one half: weights as the A operand (result rows = features:
+  // a lane holds 4 consecutive features of a token), x as B.  x operands of
+  // both 32-K parts up front, weight operands kAhead tiles ahead.
+  constexpr int kAhead = FT < 4 ? FT : 4;
+  auto compute = [&](int half) __attribute__((always_inline)) {
+    const u32x4* d = mm_lds + half * kHalf;
+    u32x4 xa[2][MT], wb[kAhead];
+#pragma unroll
+    for (int r = 0; r < MT; ++r) xa[0][r] = d[x_rd[0] + 128 * r];
+#pragma unroll
+    for (int t = 0; t < kAhead; ++t) wb[t] = d[w_rd[t / FT] + 128 * (t % FT)];
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int r = 0; r < MT; ++r) xa[1][r] = d[x_rd[1] + 128 * r];
+#pragma unroll
+    for (int t = 0; t < 2 * FT; ++t) {
+#pragma unroll
+      for (int r = 0; r < MT; ++r) acc[t % FT][r] = F16::mfma_k32(wb[t % kAhead], xa[t / FT][r], acc[t % FT][r]);
+      if (t + kAhead < 2 * FT) wb[t % kAhead] = d[w_rd[(t + kAhead) / FT] + 128 * ((t + kAhead) % FT)];
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  const bool first = wave < NW / 2;
+  load(0);
+  store(0);
+  load(1);
+  lds_barrier();
+  for (int c = 0; c < steps; ++c) {
+    const bool more = c + 1 < steps;
+    if (first && more) {
+      store((c + 1) & 1);
+      load(c + 2);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_setprio(1);
+    compute(c & 1);
+    __builtin_amdgcn_s_setprio(0);
+    __builtin_amdgcn_sched_barrier(0);
+    if (!first && more) {
+      store((c + 1) & 1);
+      load(c + 2);
+    }
+    lds_barrier();
+  }
+  // F.linear's fp16 results, staged row by row in LDS (both halves are dead),
+  // then stored as whole 8-feature pieces of rows.
+  constexpr int kPitch = BN + 8;  // fp16 values of a staged row
+  constexpr int kRowsStaged = 2 * kHalf * 8 / kPitch;  // rows the LDS holds at once
+  constexpr int kParts = kRowsStaged >= BM ? 1 : 2;
+  constexpr int kPartRows = BM / kParts;
+  static_assert(kPartRows <= kRowsStaged && kPartRows % WM == 0, "a part is whole waves' rows");
+  uint16_t* stg = reinterpret_cast<uint16_t*>(mm_lds);
+  const bool vec = reinterpret_cast<uintptr_t>(y) % 16 == 0 && y_stride % 8 == 0;
+#pragma unroll
+  for (int part = 0; part < kParts; ++part) {
+    if (part) __syncthreads();
+    if (wm * WM / kPartRows == part) {
+#pragma unroll
+      for (int f = 0; f < FT; ++f)
+#pragma unroll
+        for (int r = 0; r < MT; ++r)
+          *reinterpret_cast<u32x2*>(stg + (wm * WM % kPartRows + 16 * r + n16) * kPitch + wn * WN + 16 * f + 4 * g4) =
+              u32x2{F16::pack2(acc[f][r][0], acc[f][r][1]), F16::pack2(acc[f][r][2], acc[f][r][3])};
+    }
+    __syncthreads();
+    constexpr int kPieces = kPartRows * BN / 8;
+#pragma unroll 4
+    for (int pc = tid; pc < kPieces; pc += NT) {
+      const int r = pc / (BN / 8), col = n0 + 8 * (pc % (BN / 8)), row = m0 + part * kPartRows + r;
+      if (row >= a.m || col >= n) continue;  // n is a multiple of 16: a piece is in or out
+      const u32x4 v = *reinterpret_cast<const u32x4*>(stg + r * kPitch + 8 * (pc % (BN / 8)));
+      const int64_t off = (int64_t)row * y_stride + col;
+      if (vec && y_dtype == RIA_DT_F16) {
+        *reinterpret_cast<u32x4*>(static_cast<uint16_t*>(y) + off) = v;
+        continue;
+      }
+      float f[8];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        f[2 * e] = F16::lo_f32(v[e]);
+        f[2 * e + 1] = F16::hi_f32(v[e]);
+      }
+      if (vec && (y_add || y_dtype == RIA_DT_F32)) {
+        f32x4* yp = reinterpret_cast<f32x4*>(static_cast<float*>(y) + off);
+        f32x4 o[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          o[h] = y_add ? yp[h] : f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int e = 0; e < 4; ++e) o[h][e] = y_add ? add_rn(o[h][e], f[4 * h + e]) : f[4 * h + e];
+        }
+        yp[0] = o[0];
+        yp[1] = o[1];
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          if (y_add) {
+            float* yp = static_cast<float*>(y) + off + e;
+            *yp = add_rn(*yp, f[e]);
+          } else {
+            store_act_dt(y, off + e, f[e], y_dtype);
+          }
+        }
+      }
+    }
+  }
+}
+
 // Tile shapes of the K-split kernels (rows 16 RT, features 16 CT)
 struct KsShape {
   int rt, ct;
@@ -895,6 +1135,52 @@ static void launch_ks(const LinearArgs& a, KsShape s, dim3 grid, hipStream_t st)
     launch_ks_k<4, 4, 4, XB>(a, grid, st);
   else
     launch_ks_k<2, 2, 6, XB>(a, grid, st);
+}
+
+// Tiles of the many-row kernel (BM rows x BN features).
+struct MmShape {
+  int bm, bn;
+};
+// Fewest rows that take the many-row kernel.  A tile walks K serially, where
+// the K-split kernel's four waves share it, so the line rises with K: at K =
+// 2048, 256 rows of a layer's input projections 40.3 -> 31.7 us, 384 57.7 ->
+// 43.1 (300 rows 41.1 and 43.3); at K = 4096 and 2048 features, 1536 rows 60.1
+// -> 54.5 and 1024 rows 34.9 against 53.9.  The features do not enter: grouped
+// and separate calls must take the same kernel.
+static int mm_min_rows(int k) { return k <= 2048 ? 193 : 1345 * (k / 128) / 32; }
+
+static void launch_mm(const LinearArgs& a, MmShape s, bool xb, dim3 grid, hipStream_t st) {
+  if (s.bm == 256) {
+    if (xb)
+      hipLaunchKernelGGL((linear_fp8_mm_kernel<256, 256, 64, 128, true>), grid, dim3(512), 0, st, a);
+    else
+      hipLaunchKernelGGL((linear_fp8_mm_kernel<256, 256, 64, 128, false>), grid, dim3(512), 0, st, a);
+  } else {
+    if (xb)
+      hipLaunchKernelGGL((linear_fp8_mm_kernel<128, 128, 64, 64, true>), grid, dim3(256), 0, st, a);
+    else
+      hipLaunchKernelGGL((linear_fp8_mm_kernel<128, 128, 64, 64, false>), grid, dim3(256), 0, st, a);
+  }
+}
+
+// 256 x 256 tiles, one workgroup per CU, or 128 x 128, two: by the time of the
+// launch's rounds at K = 2048 on MI355X (a round of 256 x 256 tiles 54 us; of
+// 128 x 128 ones 30 with one per CU, 43 with two).  640 rows of a layer's
+// input projections take 47 us in small tiles and 53 in large, 777 rows 72 and
+// 58, 16384 rows 1035 and 740.
+static MmShape choose_mm(int m, int count, const ria_fp8_proj* projs) {
+  const int64_t cus = device_cus();
+  int64_t t256 = 0, t128 = 0;
+  for (int j = 0; j < count; ++j) {
+    t256 += (projs[j].n + 255) / 256;
+    t128 += (projs[j].n + 127) / 128;
+  }
+  t256 *= (m + 255) / 256;
+  t128 *= (m + 127) / 128;
+  const int64_t rest = t128 % (2 * cus);
+  const int64_t large = (t256 + cus - 1) / cus * 54;
+  const int64_t small = t128 / (2 * cus) * 43 + (rest == 0 ? 0 : rest <= cus ? 30 : 43);
+  return small < large ? MmShape{128, 128} : MmShape{256, 256};
 }
 
 static bool lin_dtype_ok(int dt) { return dt == RIA_DT_BF16 || dt == RIA_DT_F16 || dt == RIA_DT_F32; }
@@ -977,13 +1263,19 @@ static int linear_group(const char* who, int m, int k, const void* x, int x_dtyp
   // whose busiest CU moves the fewest bytes: (workgroups per CU) x (x bytes
   // + weight bytes of one workgroup); ties go to more workgroups.
   int ct = 1, mt = kLinRows;
+  MmShape mm_shape{};
   // K-split kernel (fp16 or bf16 x): the tile shape whose busiest CU moves the
   // fewest bytes, (rounds of workgroups over the CUs) x (x + weight bytes of
   // one tile)
   bool ks = !gemv && (x_dtype == RIA_DT_F16 || x_dtype == RIA_DT_BF16) && (int64_t)m * x_row_stride < (int64_t(1) << 31);
   for (int j = 0; j < count; ++j) ks = ks && (int64_t)projs[j].n * k < (int64_t(1) << 31);
   KsShape ks_shape = kKsShapes[0];
-  if (ks) {
+  const bool mm = ks && m >= mm_min_rows(k);
+  if (mm) {
+    mm_shape = choose_mm(m, count, projs);
+    ct = mm_shape.bn / 16;
+    mt = mm_shape.bm;
+  } else if (ks) {
     const int cus = device_cus();
     int64_t best = -1;
     for (const KsShape s : kKsShapes) {
@@ -1032,7 +1324,14 @@ static int linear_group(const char* who, int m, int k, const void* x, int x_dtyp
                      tile};
     tile += (q.n + 16 * ct - 1) / (16 * ct);
   }
+  a.tiles = tile;
   const int64_t mblocks = gemv ? 1 : (m + mt - 1) / mt;
+  if (mm) {
+    const int64_t wgs = (mblocks * tile + 7) / 8 * 8;
+    if (m > 65535LL * 64 || wgs > 0x7fffffff) return set_error(RIA_ERR_INVALID, "%s: too many rows", who);
+    launch_mm(a, mm_shape, x_dtype == RIA_DT_BF16, dim3(static_cast<unsigned>(wgs)), static_cast<hipStream_t>(stream));
+    return check_launch(who);
+  }
   if (mblocks > 65535) return set_error(RIA_ERR_INVALID, "%s: too many rows", who);
   const dim3 grid(static_cast<unsigned>(tile), static_cast<unsigned>(mblocks));
   hipStream_t st = static_cast<hipStream_t>(stream);

@@ -202,3 +202,38 @@ def test_linear_fp8_group_normed_host_checks(gpu):
     wn = torch.zeros((2048,), device=gpu)
     with pytest.raises(RuntimeError, match="up to 4 rows"):
         K.linear_fp8_group(x, [(w8.to(gpu), s.to(gpu))], norm_weight=wn)
+
+
+@pytest.mark.parametrize("xdt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("m,ns,k", [
+    (193, [8192, 32], 2048),            # fewest rows, 128 x 128 tiles, a 32-wide projection
+    (255, [48, 272], 128),              # two steps of K, features that end inside a tile
+    (777, [8192, 4096, 32, 32], 2048),  # 256 x 256 tiles, 9 rows past a tile
+    (4097, [272, 1040], 384),           # one row past a tile, three scale blocks of K
+    (1345, [512], 4096),                # fewest rows at K = 4096
+])
+def test_many_row_kernel(gpu, m, ns, k, xdt):
+    """Prompt-sized calls against the exact product of the same fp16 operands
+    (error within 1.5x of an fp32-accumulated product's own), grouped calls
+    equal to separate ones, the fp32 / bf16 outputs and the residual add equal
+    to the fp16 result, and nothing written past the result's columns."""
+    announce(f"linear_fp8 many rows: M={m} N={ns} K={k} x {xdt}")
+    proj = [tuple(t.to(gpu) for t in W.fp8_block_weight(800 + j, n, k)) for j, n in enumerate(ns)]
+    g = torch.Generator().manual_seed(810 + m)
+    x = torch.randn((m, k + 8), generator=g).to(xdt).to(gpu)[:, :k]
+    ys = K.linear_fp8_group(x, proj)
+    for j, (w, s) in enumerate(proj):
+        w16 = K.dequant_fp8(w, s, torch.float16)
+        exact = x.to(torch.float16).double() @ w16.double().t()
+        ref = (x.to(torch.float16).float() @ w16.float().t()).to(torch.float16)
+        e_got, e_ref = ((t.double() - exact).abs().max().item() for t in (ys[j], ref))
+        assert e_got <= 1.5 * e_ref + 1e-6, (j, e_got, e_ref)
+        wide = torch.full((m, ns[j] + 3), 7.0, device=gpu)  # rows that are not 16-byte aligned
+        K.linear_fp8(x, w, s, out=wide[:, :ns[j]])
+        assert torch.equal(wide[:, :ns[j]], ys[j].float()) and bool((wide[:, ns[j]:] == 7.0).all())
+        assert torch.equal(K.linear_fp8(x, w, s, out_dtype=torch.float32), ys[j].float())
+        assert torch.equal(K.linear_fp8(x, w, s, out_dtype=torch.bfloat16), ys[j].to(torch.bfloat16))
+        base = torch.randn((m, ns[j]), generator=g).to(gpu)
+        y = base.clone()
+        K.linear_fp8_group(x, [(w, s)], out=[y], accumulate=[True])
+        assert torch.equal(y, base + ys[j].float())
