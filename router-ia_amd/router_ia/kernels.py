@@ -29,12 +29,17 @@ def dtype_code(t: torch.Tensor) -> int:
         raise TypeError(f"unsupported activation dtype {t.dtype}; expected bf16, fp16 or fp32") from None
 
 
-def _ptr(t: torch.Tensor | None) -> ctypes.c_void_p | None:
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+# The helpers below run for every tensor of every call, and a decode step of a
+# small batch is shorter on the GPU than its calls on the host (a DeltaNet
+# layer at batch 1: 6.7 us of kernel, 24 us of Python).  So they look at plain
+# ints (get_device, strides, raw stream handles) and build no device, stream,
+# view or ctypes objects unless something is wrong.
+def _ptr(t: torch.Tensor | None) -> int | None:
+    return None if t is None else t.data_ptr()
 
 
 def _require_gpu(name: str, t: torch.Tensor | None, device: torch.device | None = None) -> None:
-    if t is None:
+    if t is None or (t.is_cuda and (device is None or t.get_device() == device.index)):
         return
     if t.device.type != "cuda":
         raise RuntimeError(
@@ -44,8 +49,9 @@ def _require_gpu(name: str, t: torch.Tensor | None, device: torch.device | None 
         raise RuntimeError(f"{name} is on {t.device}, expected {device}")
 
 
-def _stream(device: torch.device) -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+def _stream(device: torch.device) -> int:
+    index = device.index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
 
 
 def _rows_i32(name: str, t: torch.Tensor | int | None, batch: int, device: torch.device) -> tuple[torch.Tensor | None, int]:
@@ -62,6 +68,20 @@ def _rows_i32(name: str, t: torch.Tensor | int | None, batch: int, device: torch
 
 def _row_stride(name: str, t: torch.Tensor, batch: int, row_elems: int) -> int:
     """Row stride (elements) of a [batch, ...] tensor whose rows are contiguous."""
+    shape = t.shape
+    if len(shape) < 2 or shape[0] != batch or batch == 0:
+        return _row_stride_checked(name, t, batch, row_elems)
+    strides, run = t.stride(), 1
+    for d in range(len(shape) - 1, 0, -1):
+        if strides[d] != run and shape[d] != 1:
+            return _row_stride_checked(name, t, batch, row_elems)
+        run *= shape[d]
+    if run != row_elems:
+        return _row_stride_checked(name, t, batch, row_elems)
+    return strides[0] if batch > 1 else row_elems
+
+
+def _row_stride_checked(name: str, t: torch.Tensor, batch: int, row_elems: int) -> int:
     flat = t.reshape(t.shape[0], -1) if t.dim() > 2 else t
     if flat.dim() != 2 or flat.shape[0] != batch or flat.shape[1] != row_elems:
         raise ValueError(f"{name} must have {batch} rows of {row_elems} elements, got {tuple(t.shape)}")
@@ -76,7 +96,7 @@ def conv_dim(num_k_heads: int, num_v_heads: int) -> int:
     return (2 * num_k_heads + num_v_heads) * GDN_HEAD_DIM
 
 
-def _norm_weight(name: str, w: torch.Tensor | None, n: int, dev: torch.device) -> ctypes.c_void_p | None:
+def _norm_weight(name: str, w: torch.Tensor | None, n: int, dev: torch.device) -> int | None:
     """A norm weight as the ABI takes it: contiguous fp32 [n] on the device (16-byte aligned)."""
     if w is None:
         return None
@@ -121,7 +141,7 @@ def gdn_decode(
                     ("A_log", A_log), ("dt_bias", dt_bias)):
         _require_gpu(name, t, dev)
     x_stride = _row_stride("mixed_qkv", mixed_qkv, batch, cdim)
-    if state.dtype != torch.float32 or state.dim() != 4 or tuple(state.shape[1:]) != (num_v_heads, 128, 128) \
+    if state.dtype != torch.float32 or state.dim() != 4 or state.shape[1:] != (num_v_heads, 128, 128) \
             or not state.is_contiguous():
         raise ValueError(f"state must be contiguous fp32 [pool, {num_v_heads}, 128, 128], got {tuple(state.shape)}")
     if seq_slot is None and state.shape[0] < batch:
@@ -131,7 +151,7 @@ def gdn_decode(
     g_stride = _row_stride("gate_a", gate_a, batch, num_v_heads)
     if _row_stride("gate_b", gate_b, batch, num_v_heads) != g_stride:
         raise ValueError("gate_a and gate_b must share a row stride")
-    if tuple(out.shape) != (batch, num_v_heads, GDN_HEAD_DIM) or not out.is_contiguous():
+    if out.shape != (batch, num_v_heads, GDN_HEAD_DIM) or not out.is_contiguous():
         raise ValueError(f"out must be contiguous [{batch}, {num_v_heads}, 128]")
     if fuse_conv:
         if conv_weight is None or conv_ring is None:
@@ -222,7 +242,7 @@ def gdn_decode_ex(
     g_stride = _row_stride("gate_a", gate_a, batch, num_v_heads)
     if _row_stride("gate_b", gate_b, batch, num_v_heads) != g_stride:
         raise ValueError("gate_a and gate_b must share a row stride")
-    if tuple(out.shape) != (batch, num_v_heads, GDN_HEAD_DIM) or not out.is_contiguous():
+    if out.shape != (batch, num_v_heads, GDN_HEAD_DIM) or not out.is_contiguous():
         raise ValueError(f"out must be contiguous [{batch}, {num_v_heads}, 128]")
     if conv_layout == nat.RIA_CONV_RING:
         if conv_weight is None or conv_ring is None:
@@ -267,7 +287,7 @@ def gdn_decode_ex(
         A_log=addr(A_log) if gate_mode == nat.RIA_GATE_RAW else None,
         dt_bias=addr(dt_bias) if gate_mode == nat.RIA_GATE_RAW else None, qk_mode=int(qk_mode), out=addr(out),
         out_dtype=dtype_code(out), z=addr(z), z_dtype=dtype_code(z) if z is not None else 0, z_row_stride=z_stride,
-        norm_weight=w_ptr.value if w_ptr is not None else None, pool_rows=int(state_in.shape[0]))
+        norm_weight=w_ptr, pool_rows=int(state_in.shape[0]))
     rc = nat.load().ria_gdn_decode_ex(ctypes.byref(d), _stream(dev))
     nat.check(rc, "ria_gdn_decode_ex")
     return out
@@ -296,7 +316,7 @@ def conv1d_window_step(x: torch.Tensor, conv_weight: torch.Tensor, window_in: to
         _require_gpu(name, t, dev)
     stride = _row_stride("x", x, batch, channels)
     _check_conv_window(conv_weight, window_in, window_out, channels, batch)
-    if tuple(out.shape) != (batch, channels) or not out.is_contiguous():
+    if out.shape != (batch, channels) or not out.is_contiguous():
         raise ValueError(f"out must be contiguous [{batch}, {channels}]")
     rc = nat.load().ria_conv1d_window_step(batch, channels, _ptr(x), dtype_code(x), stride, _ptr(conv_weight),
                                            _ptr(window_in), _ptr(window_out), _ptr(out), dtype_code(out),
@@ -333,7 +353,7 @@ def conv1d_step(
         _require_gpu(name, t, dev)
     stride = _row_stride("x", x, batch, channels)
     _check_conv_tensors(conv_weight, conv_ring, channels, batch if seq_slot is None else 0)
-    if tuple(out.shape) != (batch, channels) or not out.is_contiguous():
+    if out.shape != (batch, channels) or not out.is_contiguous():
         raise ValueError(f"out must be contiguous [{batch}, {channels}]")
     if seq_slot is not None:
         _rows_i32("seq_slot", seq_slot, batch, dev)
@@ -461,9 +481,9 @@ KV_DTYPES = (torch.bfloat16, torch.float16)
 def _check_kv_cache(k_cache: torch.Tensor, v_cache: torch.Tensor, num_kv_heads: int) -> int:
     if k_cache.dtype not in KV_DTYPES or v_cache.dtype != k_cache.dtype:
         raise ValueError("KV caches must both be bf16 or both fp16")
-    if k_cache.dim() != 6 or tuple(k_cache.shape[1:]) != (num_kv_heads, *K_TILE_SHAPE):
+    if k_cache.dim() != 6 or k_cache.shape[1:] != (num_kv_heads, *K_TILE_SHAPE):
         raise ValueError(f"k_cache must be [pages, {num_kv_heads}, 8, 4, 16, 8], got {tuple(k_cache.shape)}")
-    if v_cache.dim() != 4 or tuple(v_cache.shape[1:]) != (num_kv_heads, ATTN_HEAD_DIM, PAGE_TOKENS):
+    if v_cache.dim() != 4 or v_cache.shape[1:] != (num_kv_heads, ATTN_HEAD_DIM, PAGE_TOKENS):
         raise ValueError(f"v_cache must be [pages, {num_kv_heads}, 256, 16], got {tuple(v_cache.shape)}")
     if k_cache.shape[0] != v_cache.shape[0] or not k_cache.is_contiguous() or not v_cache.is_contiguous():
         raise ValueError("k_cache / v_cache must be contiguous with equal page counts")
@@ -584,7 +604,7 @@ def attn_decode(
         raise ValueError(f"max_ctx {max_ctx} exceeds the page table capacity {page_table.shape[1] * PAGE_TOKENS}")
     if seq_slot is None and page_table.shape[0] < batch:
         raise ValueError("page table has fewer rows than batch")
-    if tuple(out.shape) != (batch, num_q_heads, ATTN_HEAD_DIM) or not out.is_contiguous():
+    if out.shape != (batch, num_q_heads, ATTN_HEAD_DIM) or not out.is_contiguous():
         raise ValueError(f"out must be contiguous [{batch}, {num_q_heads}, 256]")
     if not workspace.is_contiguous():
         raise ValueError("workspace must be contiguous")
@@ -640,9 +660,9 @@ def _fp8_weight(name: str, w: torch.Tensor, scale_inv: torch.Tensor, dev: torch.
     _require_gpu(name + " scale_inv", scale_inv, dev)
     if w.dtype not in (torch.float8_e4m3fn, torch.uint8) or w.dim() != 2 or not w.is_contiguous():
         raise ValueError(f"{name} must be a contiguous float8_e4m3fn (or its uint8 bytes) [N, K] tensor")
-    n, k = int(w.shape[0]), int(w.shape[1])
+    n, k = w.shape
     grid = ((n + FP8_BLOCK - 1) // FP8_BLOCK, (k + FP8_BLOCK - 1) // FP8_BLOCK)
-    if scale_inv.dtype != torch.float32 or tuple(scale_inv.shape) != grid or not scale_inv.is_contiguous():
+    if scale_inv.dtype != torch.float32 or scale_inv.shape != grid or not scale_inv.is_contiguous():
         raise ValueError(f"{name} scale_inv must be contiguous fp32 {grid}, got {tuple(scale_inv.shape)}")
     return n, k
 
@@ -709,20 +729,24 @@ def linear_fp8_group(x: torch.Tensor, projections: list[tuple[torch.Tensor, torc
         raise ValueError(f"x must be [M, {k}] with contiguous rows, got {tuple(x.shape)}")
     m = int(x.shape[0])
     xs = int(x.stride(0)) if m > 1 else k
-    if out is None:
+    given = out is not None
+    if not given:
         dts = out_dtype if isinstance(out_dtype, (list, tuple)) else [out_dtype] * len(shapes)
         out = [torch.empty((m, n), dtype=dt, device=dev) for (n, _), dt in zip(shapes, dts)]
     if len(out) != len(projections):
         raise ValueError("out must hold one tensor per projection")
     arr = (nat.Fp8Proj * len(projections))()
     for j, ((w, s), (n, _), y) in enumerate(zip(projections, shapes, out)):
-        _require_gpu(f"out {j}", y, dev)
-        if y.dim() != 2 or tuple(y.shape) != (m, n) or (n > 1 and y.stride(1) != 1):
-            raise ValueError(f"out {j} must be [{m}, {n}] with contiguous rows")
+        if given:
+            _require_gpu(f"out {j}", y, dev)
+            if y.dim() != 2 or y.shape != (m, n) or (n > 1 and y.stride(1) != 1):
+                raise ValueError(f"out {j} must be [{m}, {n}] with contiguous rows")
         add = bool(accumulate[j]) if accumulate is not None else False
         if add and y.dtype != torch.float32:
             raise ValueError(f"out {j}: accumulating needs fp32")
-        arr[j] = nat.Fp8Proj(_ptr(w), _ptr(s), _ptr(y), int(y.stride(0)) if m > 1 else n, n, dtype_code(y), int(add))
+        p = arr[j]
+        p.weight, p.scale_inv, p.y = w.data_ptr(), s.data_ptr(), y.data_ptr()
+        p.y_row_stride, p.n, p.y_dtype, p.y_add = y.stride(0) if m > 1 else n, n, dtype_code(y), add
     if norm_weight is None:
         rc = nat.load().ria_linear_fp8_group(m, k, _ptr(x), dtype_code(x), xs, len(projections),
                                              ctypes.addressof(arr), _stream(dev))
@@ -829,7 +853,7 @@ def gdn_prefill(
                     ("A_log", A_log), ("dt_bias", dt_bias)):
         _require_gpu(name, t, dev)
     xs = _row_stride("mixed_qkv", mixed_qkv, length, cdim)
-    if state.dtype != torch.float32 or tuple(state.shape) != (num_v_heads, 128, 128) or not state.is_contiguous():
+    if state.dtype != torch.float32 or state.shape != (num_v_heads, 128, 128) or not state.is_contiguous():
         raise ValueError(f"state must be contiguous fp32 [{num_v_heads}, 128, 128]")
     _check_conv_tensors(conv_weight, conv_ring.reshape(1, CONV_RING, cdim), cdim, 1)
     if gate_a.dtype != torch.float32 or gate_b.dtype != torch.float32:
@@ -837,7 +861,7 @@ def gdn_prefill(
     gs = _row_stride("gate_a", gate_a, length, num_v_heads)
     if _row_stride("gate_b", gate_b, length, num_v_heads) != gs:
         raise ValueError("gate_a and gate_b must share a row stride")
-    if tuple(out.shape) != (length, num_v_heads, GDN_HEAD_DIM) or not out.is_contiguous():
+    if out.shape != (length, num_v_heads, GDN_HEAD_DIM) or not out.is_contiguous():
         raise ValueError(f"out must be contiguous [{length}, {num_v_heads}, 128]")
     if gate_mode == nat.RIA_GATE_RAW:
         for name, t in (("A_log", A_log), ("dt_bias", dt_bias)):
@@ -971,7 +995,7 @@ def _attn_decode_append(q, gate, k, v, k_cache, v_cache, page_table, out, *, pos
         raise ValueError(f"max_ctx {max_ctx} exceeds the page table capacity {page_table.shape[1] * PAGE_TOKENS}")
     if seq_slot is None and page_table.shape[0] < batch:
         raise ValueError("page table has fewer rows than batch")
-    if tuple(out.shape) != (batch, num_q_heads, ATTN_HEAD_DIM) or not out.is_contiguous():
+    if out.shape != (batch, num_q_heads, ATTN_HEAD_DIM) or not out.is_contiguous():
         raise ValueError(f"out must be contiguous [{batch}, {num_q_heads}, 256]")
     if workspace is not None and not workspace.is_contiguous():
         raise ValueError("workspace must be contiguous")
@@ -1084,7 +1108,7 @@ def attn_prefill(
     if out is None:
         out = torch.empty((length, num_q_heads, ATTN_HEAD_DIM), device=dev, dtype=q.dtype)
     _require_gpu("out", out, dev)
-    if tuple(out.shape) != (length, num_q_heads, ATTN_HEAD_DIM) or not out.is_contiguous() or out.dtype != q.dtype:
+    if out.shape != (length, num_q_heads, ATTN_HEAD_DIM) or not out.is_contiguous() or out.dtype != q.dtype:
         raise ValueError(f"out must be contiguous [{length}, {num_q_heads}, 256] of q's dtype")
     rope_dim = 0 if inv_freq is None else 2 * int(inv_freq.numel())
     head = (length, num_q_heads, num_kv_heads, _ptr(q), qs, _ptr(k), ks, _ptr(v), vs, _ptr(gate), gs, dtype_code(q),
