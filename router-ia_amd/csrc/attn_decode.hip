@@ -348,14 +348,15 @@ constexpr int kMaxBalancedUnits = 4096;
 constexpr int kMinChunkPages = 4;  // 64 tokens: small batches still spread over the CUs
 constexpr int kPadUnitsRatio = 32;
 
-// Inclusive scan of one value per lane over a wave.
+// Inclusive scan of one value per lane over a wave (DPP shifts within rows of
+// 16 lanes, then the rows' totals broadcast into the later rows).
 __device__ __forceinline__ int wave_inclusive_scan(int v) {
-  const int lane = threadIdx.x & 63;
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    const int y = __shfl_up(v, off, 64);
-    if (lane >= off) v += y;
-  }
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);   // row_shr:1
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true);   // row_shr:2
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true);   // row_shr:4
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true);   // row_shr:8
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast:15 into rows 1 and 3
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast:31 into rows 2 and 3
   return v;
 }
 
@@ -363,12 +364,7 @@ __device__ __forceinline__ int wave_inclusive_scan(int v) {
 // the exclusive prefix of this thread's value and the block total.
 __device__ int block_exclusive_scan(int v, int* scratch, int* total) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  int x = v;
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    const int y = __shfl_up(x, off, 64);
-    if (lane >= off) x += y;
-  }
+  const int x = wave_inclusive_scan(v);
   if (lane == 63) scratch[wave] = x;
   lds_barrier();
   int base = 0;
@@ -553,8 +549,7 @@ __global__ __launch_bounds__(256, 2) void attn_splitk_kernel(AttnArgs a) {
         sc[i] = (t_base + i < tok1) ? sc[i] * sl2 : -INFINITY;
         mx = fmaxf(mx, sc[i]);
       }
-      mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+      mx = quad_row_max(mx);
       // Lazy rescale: keep the reference max while the page max stays within
       // 2^8 of it, so the accumulator is rescaled only when it has to be.
       const bool grow = mx > m_run + 8.0f;
@@ -623,8 +618,7 @@ __global__ __launch_bounds__(256, 2) void attn_splitk_kernel(AttnArgs a) {
         p = pn;
       }
     }
-    l_run += __shfl_xor(l_run, 16, 64);
-    l_run += __shfl_xor(l_run, 32, 64);
+    l_run = add_xor<32>(add_xor<16>(l_run));
 
     // ---- merge the four waves through LDS (q_lds is dead: every wave passed the barrier above)
     if (g4 == 0 && n < G) {

@@ -26,6 +26,7 @@
 // exactly once with full-row coalescing.  The two column reductions over i
 // (r_j and the S' q part of o_j) share a single shuffle + LDS pass.
 #include <algorithm>
+#include <type_traits>
 
 #include "ria_common.h"
 
@@ -266,14 +267,17 @@ __global__ __launch_bounds__(256) void gdn_decode_kernel(GdnDecodeArgs a) {
       oj[c] = fmaf(s[r][c], qi, oj[c]);
     }
   }
-#pragma unroll
-  for (int off = TPR; off < 64; off <<= 1) {
+  auto add_rows = [&](auto off) {  // lanes that hold the same columns
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
-      rj[c] += __shfl_xor(rj[c], off, 64);
-      oj[c] += __shfl_xor(oj[c], off, 64);
+      rj[c] = add_xor<decltype(off)::value>(rj[c]);
+      oj[c] = add_xor<decltype(off)::value>(oj[c]);
     }
-  }
+  };
+  if constexpr (TPR <= 4) add_rows(std::integral_constant<int, 4>{});
+  if constexpr (TPR <= 8) add_rows(std::integral_constant<int, 8>{});
+  if constexpr (TPR <= 16) add_rows(std::integral_constant<int, 16>{});
+  if constexpr (TPR <= 32) add_rows(std::integral_constant<int, 32>{});
   if (lane < TPR) {
 #pragma unroll
     for (int c = 0; c < 4; ++c) {

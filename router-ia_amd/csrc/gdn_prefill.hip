@@ -440,10 +440,8 @@ __global__ __launch_bounds__(256, 3) void chunk_prep_kernel(PrefillArgs a) {
       sq += mul_rn(qv[s][j], qv[s][j]);
       sk += mul_rn(kv[s][j], kv[s][j]);
     }
-  sq += __shfl_xor(sq, 16, 64);
-  sq += __shfl_xor(sq, 32, 64);
-  sk += __shfl_xor(sk, 16, 64);
-  sk += __shfl_xor(sk, 32, 64);
+  sq = add_xor<32>(add_xor<16>(sq));
+  sk = add_xor<32>(add_xor<16>(sk));
   const float iq = 1.0f / sqrtf(sq + 1e-6f), ik = 1.0f / sqrtf(sk + 1e-6f);
   // No barrier here: beta_s and G_s are first read in step 3, after the next
   // one, and until then each wave writes only its own rows.

@@ -376,10 +376,45 @@ constexpr int kBufferWord3 = 0x00020000;
 
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
-  return v;
+// v + (v of lane ^ OFF), in lane exchanges of a few cycles (permlane swaps and
+// DPP; xor 4, which has no such form, by ds_swizzle) instead of an LDS permute
+// round trip.  All lanes must be active.
+template <int OFF>
+__device__ __forceinline__ float add_xor(float v) {
+  if constexpr (OFF == 32 || OFF == 16) {
+    const uint32_t u = __float_as_uint(v);
+    const auto r = OFF == 32 ? __builtin_amdgcn_permlane32_swap(u, u, false, false)
+                             : __builtin_amdgcn_permlane16_swap(u, u, false, false);
+    return add_rn(__uint_as_float(r[0]), __uint_as_float(r[1]));
+  } else if constexpr (OFF == 4) {
+    return add_rn(v, __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(v), 0x1f | (4 << 10))));
+  } else {
+    static_assert(OFF == 8 || OFF == 2 || OFF == 1, "a lane bit");
+    constexpr int kCtrl = OFF == 8 ? 0x128 : OFF == 2 ? 0x4E : 0xB1;  // row_ror:8, quad_perm [2,3,0,1], [1,0,3,2]
+    return add_rn(v, __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), kCtrl, 0xf, 0xf, true)));
+  }
+}
+
+// Sum over each group of RL lanes, added in the order xor RL / 2, .., 2, 1.
+// After the xor 8 step lanes 8 apart agree, so a rotation by 4 is the xor 4.
+template <int RL>
+__device__ __forceinline__ float group_sum(float v) {
+  static_assert(RL == 64 || RL == 32 || RL == 16, "16 lanes or more");
+  if constexpr (RL >= 64) v = add_xor<32>(v);
+  if constexpr (RL >= 32) v = add_xor<16>(v);
+  v = add_xor<8>(v);
+  v = add_rn(v, __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x124, 0xf, 0xf, true)));  // row_ror:4
+  return add_xor<1>(add_xor<2>(v));
+}
+
+__device__ __forceinline__ float wave_sum(float v) { return group_sum<64>(v); }
+
+// max(v, v of lane ^ 16 and ^ 32): the four lanes that share lane % 16.
+__device__ __forceinline__ float quad_row_max(float v) {
+  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  const float m = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+  const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(m), __float_as_uint(m), false, false);
+  return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
 }
 
 // Sum over each half of the wavefront (lanes 0..31 and 32..63 separately),

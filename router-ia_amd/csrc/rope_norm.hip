@@ -155,8 +155,7 @@ __global__ __launch_bounds__(256) void rmsnorm_vec_kernel(NormArgs a) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) ss = add_rn(ss, mul_rn(v[q][j], v[q][j]));
     }
-#pragma unroll
-    for (int off = RL / 2; off >= 1; off >>= 1) ss += __shfl_xor(ss, off, 64);
+    ss = group_sum<RL>(ss);
     if (!ok) return;
     const float rs = rms_scale(ss, a.dim, a.eps);
 #pragma unroll
@@ -170,8 +169,7 @@ __global__ __launch_bounds__(256) void rmsnorm_vec_kernel(NormArgs a) {
         for (int j = 0; j < 4; ++j) ss = add_rn(ss, mul_rn(v[j], v[j]));
       }
     }
-#pragma unroll
-    for (int off = RL / 2; off >= 1; off >>= 1) ss += __shfl_xor(ss, off, 64);
+    ss = group_sum<RL>(ss);
     if (!ok) return;
     const float rs = rms_scale(ss, a.dim, a.eps);
     for (int c = 4 * li; c < a.dim; c += 4 * RL) {
