@@ -196,45 +196,38 @@ __global__ __launch_bounds__(kPrefillThreads) __attribute__((amdgpu_waves_per_eu
     const bool row_ok = head_ok && t_row < a.length;
     const int qpos = a.start + t_row;
     const int64_t base = (int64_t)t_row * a.q_stride + (int64_t)head * kAttnHeadDim + 8 * g4;
-    auto load_q8 = [&](int kd, float (&y)[8]) {
+    auto load_q8 = [&](int kd, float (&x)[8]) {
       if (row_ok) {
-        load_act8<AT>(a.q, base + 32 * kd, y);
+        load_act8<AT>(a.q, base + 32 * kd, x);
       } else {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) y[j] = 0.f;
+        for (int j = 0; j < 8; ++j) x[j] = 0.f;
       }
     };
-    // q_norm (qwen36_attention_cache.py:302-304) before RoPE: a first pass
-    // for the row's sum of squares, whose four 64-dim slices sit in lanes
-    // n, n + 16, n + 32, n + 48; the second pass normalises as it loads.
-    float qs = 1.f;
+    float y[8][8];
+#pragma unroll
+    for (int kd = 0; kd < 8; ++kd) load_q8(kd, y[kd]);
+    // q_norm (qwen36_attention_cache.py:302-304) before RoPE: the row's sum of
+    // squares, whose four 64-dim slices sit in lanes n, n + 16, n + 32, n + 48.
     if (a.q_norm_w) {
       float ss = 0.f;
 #pragma unroll
-      for (int kd = 0; kd < 8; ++kd) {
-        float y[8];
-        load_q8(kd, y);
+      for (int kd = 0; kd < 8; ++kd)
 #pragma unroll
-        for (int j = 0; j < 8; ++j) ss = add_rn(ss, mul_rn(y[j], y[j]));
-      }
-      qs = rms_scale(swap_sum(swap_sum(ss, true), false), kAttnHeadDim);
-    }
-    auto load_qn = [&](int kd, float (&y)[8]) {
-      load_q8(kd, y);
-      if (a.q_norm_w) {
+        for (int j = 0; j < 8; ++j) ss = add_rn(ss, mul_rn(y[kd][j], y[kd][j]));
+      const float qs = rms_scale(swap_sum(swap_sum(ss, true), false), kAttnHeadDim);
+#pragma unroll
+      for (int kd = 0; kd < 8; ++kd) {
         const f32x4* wp = reinterpret_cast<const f32x4*>(a.q_norm_w + 32 * kd + 8 * g4);
         const f32x4 w0 = wp[0], w1 = wp[1];
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-          y[j] = rmsnorm_elem<AT>(y[j], qs, w0[j]);
-          y[4 + j] = rmsnorm_elem<AT>(y[4 + j], qs, w1[j]);
+          y[kd][j] = rmsnorm_elem<AT>(y[kd][j], qs, w0[j]);
+          y[kd][4 + j] = rmsnorm_elem<AT>(y[kd][4 + j], qs, w1[j]);
         }
       }
-    };
+    }
     // dims [0, 64) are kd 0, 1; rotate_half pairs dim 8 g4 + j with 32 + 8 g4 + j
-    float x[2][8];
-#pragma unroll
-    for (int kd = 0; kd < 2; ++kd) load_qn(kd, x[kd]);
     if (a.rope_dim == 64) {
       const float pos = static_cast<float>(qpos);
 #pragma unroll
@@ -242,24 +235,16 @@ __global__ __launch_bounds__(kPrefillThreads) __attribute__((amdgpu_waves_per_eu
         const float ang = mul_rn(pos, a.inv_freq[8 * g4 + j]);
         float cs, sn;
         sincosf(ang, &sn, &cs);
-        const float x1 = x[0][j], x2 = x[1][j];
-        x[0][j] = add_rn(mul_rn(x1, cs), mul_rn(-x2, sn));
-        x[1][j] = add_rn(mul_rn(x2, cs), mul_rn(x1, sn));
+        const float x1 = y[0][j], x2 = y[1][j];
+        y[0][j] = add_rn(mul_rn(x1, cs), mul_rn(-x2, sn));
+        y[1][j] = add_rn(mul_rn(x2, cs), mul_rn(x1, sn));
       }
     }
 #pragma unroll
-    for (int kd = 0; kd < 2; ++kd) {
+    for (int kd = 0; kd < 8; ++kd) {
 #pragma unroll
-      for (int j = 0; j < 8; ++j) x[kd][j] *= sl2;
-      pack(x[kd], qh[c][kd], ql[kd], std::true_type{});
-    }
-#pragma unroll
-    for (int kd = 2; kd < 8; ++kd) {
-      float y[8];
-      load_qn(kd, y);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) y[j] *= sl2;
-      pack(y, qh[c][kd], ql[kd], std::true_type{});
+      for (int j = 0; j < 8; ++j) y[kd][j] *= sl2;
+      pack(y[kd], qh[c][kd], ql[kd], std::true_type{});
     }
   }
 
