@@ -113,7 +113,6 @@ class BatchedAttentionState:
         self.prefill_segment_tokens = max(64, int(prefill_segment_tokens))
         self.prefill_workspace: torch.Tensor | None = None
         self.prefill_stage: torch.Tensor | None = None  # fp16 keys of a prompt from slot 0 (attention prefill)
-        self.prefill_partials: torch.Tensor | None = None  # split keys of a short prompt (attention prefill)
 
     def _size_workspace(self) -> None:
         ws = K.attn_decode_workspace_bytes(self.max_seqs, self.num_q_heads, self.num_kv_heads, self.max_context,
@@ -285,14 +284,14 @@ class BatchedAttentionState:
         # a prompt that starts the row attends over fp16 copies of its own keys (the stage)
         length = int(q.shape[0])
         stage = self._prefill_stage(length) if start == 0 else None
+        # partial sums of split query blocks: allocated per call, so that rows may run on several streams
         need = K.prefill_attn_workspace_bytes(length, self.num_q_heads, self.num_kv_heads, start,
                                               stage is not None or self.kv.dtype == torch.float16)
-        if need and (self.prefill_partials is None or self.prefill_partials.numel() < need):
-            self.prefill_partials = torch.empty(need, dtype=torch.uint8, device=self.device)
+        partials = torch.empty(need, dtype=torch.uint8, device=self.device) if need else None
         return K.attn_prefill(q, k, v, gate, k_cache, v_cache, self.kv.page_table[row], out,
                               start=start, inv_freq=self.inv_freq, scale=self.scale,
                               q_norm_weight=q_norm_weight, k_norm_weight=k_norm_weight, stage=stage,
-                              workspace=self.prefill_partials if need else None)
+                              workspace=partials)
 
     def _prefill_stage(self, length: int) -> torch.Tensor:
         need = K.prefill_stage_bytes(length, self.num_kv_heads)
