@@ -142,12 +142,16 @@ __device__ __forceinline__ void load8(const float* p, float* v) {
 // form at about a third of its instructions, and the tile path addresses rows
 // through buffer resources with the row in the scalar offset (146 -> 125 us).
 // A launch of few 64-token tiles leaves too few waves to cover the loads of
-// the next tile with the arithmetic of this one, so it takes tiles of 16
-// (three history rows read per 16): 46.7 -> 36.4 us at 4096 tokens (1024
-// tiles of 64), 36 -> 9.8 us at 300 with the gate pass below; tiles of 64 take
-// 31 us per 4096 tokens in one 16384-token launch, where they stay.
-constexpr int kConvShortTile = 16;
-constexpr int kConvTileWgs = 2048;  // fewer 64-token tiles than this: short tiles
+// the next tile with the arithmetic of this one, and a tile's tokens are a
+// serial chain, so short segments take short tiles (three history rows read
+// per tile).  Kernel times on MI355X in tiles of 16 / 8 / 4 tokens: 64 tokens
+// 6.7 / 5.1 / 4.5 us, 300 tokens 9.4 / 8.0 / 6.4, 1024 tokens 13.7 / 12.0 /
+// 11.5, 2048 20.0 / 18.8 / 19.0, 3072 29.1 / 28.5 / 35.6, 4096 36.5 / 37.0 /
+// 48.0 (46.7 in tiles of 64); tiles of 64 take 31 us per 4096 tokens in one
+// 16384-token launch, where they stay.
+constexpr int kConvShortTile = 8, kConvShortestTile = 4;
+constexpr int kConvTileWgs = 2048;     // fewer 64-token tiles (x 512 channels) than this: short tiles
+constexpr int kConvShortestWgs = 512;  // .. at most this: the shortest (2048 tokens of 8192 channels)
 
 // Gate pass (the conv launch's workgroup columns past the channels): one wave
 // per (chunk cl, V head h), lane t token t of the chunk.  beta =
@@ -1077,13 +1081,15 @@ extern "C" int ria_gdn_prefill(int length, int num_k_heads, int num_v_heads, con
     a.tok0 = c0 * kChunk;
     a.seg_tokens = min(a.seg_chunks * kChunk, length - a.tok0);
     a.conv_cols = (conv_dim / 2 + 255) / 256;
-    const bool short_tiles = a.conv_cols * a.seg_chunks < kConvTileWgs;
-    const int tiles = short_tiles ? kChunk / kConvShortTile : 1;  // per chunk
+    const int wgs = a.conv_cols * a.seg_chunks;
+    const int tiles = kChunk / (wgs <= kConvShortestWgs ? kConvShortestTile : wgs < kConvTileWgs ? kConvShortTile : kChunk);
     dim3 cgrid(a.conv_cols + ((num_v_heads + 3) / 4 + tiles - 1) / tiles, a.seg_chunks * tiles);
     dim3 pgrid(num_v_heads, a.seg_chunks);
     dim3 sgrid(num_v_heads * (kDim / 16));
 #define RIA_PREFILL_PHASES(XT_)                                                                          \
-  if (short_tiles)                                                                                       \
+  if (tiles == kChunk / kConvShortestTile)                                                               \
+    hipLaunchKernelGGL((prefill_conv_kernel<XT_, kConvShortestTile>), cgrid, dim3(256), 0, st, a);       \
+  else if (tiles == kChunk / kConvShortTile)                                                             \
     hipLaunchKernelGGL((prefill_conv_kernel<XT_, kConvShortTile>), cgrid, dim3(256), 0, st, a);          \
   else                                                                                                   \
     hipLaunchKernelGGL((prefill_conv_kernel<XT_, kChunk>), cgrid, dim3(256), 0, st, a);                  \

@@ -207,7 +207,7 @@ def test_prefill_conv_load_paths_agree(gpu):
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("length", [15, 16, 17, 79, 129])
 def test_prefill_conv_short_tiles(gpu, dtype, length):
-    """Prompts that end around the conv's 16-token tiles and inside a chunk:
+    """Prompts that end around the conv's short tiles and inside a chunk:
     16-bit rows loaded in pairs against the per-channel path (odd row stride),
     the same bits, and the oracle on the same 16-bit inputs."""
     announce(f"gdn_prefill: {dtype} conv tiles, {length} tokens")
@@ -226,3 +226,16 @@ def test_prefill_conv_short_tiles(gpu, dtype, length):
     want, s_want, _ = _oracle_tokens(params, inputs, length, state0[None], ring_to_window(ring0, 6))
     assert_act_close(got[0], want, "outputs vs oracle")
     assert_state_close(got[1][None], s_want, "final state vs oracle")
+
+
+@pytest.mark.parametrize("length", [2045, 2051, 2113])
+def test_prefill_conv_tile_lengths_agree(gpu, length):
+    """Prompts around 2048 tokens take conv tiles of 4 or 8 tokens in one pass
+    and of 4 in segments of 512: the same bits."""
+    announce(f"gdn_prefill: conv tiles of one pass vs 512-token segments, {length} tokens")
+    params = W.gdn_layer_params(71)
+    inputs = W.gdn_step_inputs(72, length, 1)
+    state0, ring0 = _init(73)
+    whole = _gpu_prefill(gpu, params, inputs, length, state0, ring0, 9)
+    parts = _gpu_prefill(gpu, params, inputs, length, state0, ring0, 9, ws_tokens=512)
+    assert all(torch.equal(x, y) for x, y in zip(whole, parts))
