@@ -31,8 +31,8 @@
 //                        turned into MFMA operands through each wave's own
 //                        LDS region.
 //   linear_fp8_mm_kernel prompts (a few hundred rows and more): tiles of 256 x
-//                        256 or 128 x 128 over the whole K, both operands
-//                        converted once into a double buffer in LDS.
+//                        256, 256 x 128 or 128 x 128 over the whole K, both
+//                        operands converted once into a double buffer in LDS.
 #include <algorithm>
 #include <type_traits>
 #include <utility>
@@ -847,36 +847,41 @@ __global__ __launch_bounds__(64 * NW) void linear_fp8_ks_kernel(const LinearArgs
 }
 
 // Many rows (prompts): tiles of BM rows x BN features over the whole of K, 64
-// K a step, two wave groups.  Per step the workgroup's threads load x (fp16,
+// K (a chunk) a step, two wave groups.  Per step the workgroup's threads load x (fp16,
 // or bf16: XB) and fp8 weights row-contiguously into registers, convert them
 // once (weights to fp16(w8 s), the same values as every kernel here) and write
 // them to one half of a double buffer in LDS in MFMA operand order, while the
-// MFMAs read the other half; one barrier a step.  A tile of 256 x 256
+// MFMAs read the other half; one barrier a step.  A tile of 256 rows
 // dequantises a weight once per 256 rows (the K-split kernel once per 64, which
-// made it VALU-bound: 25 M weights x 256 row blocks at 16384 rows) and each
-// wave's 64 x 128 of results takes 24 operand reads for 64 MFMAs.  The two
+// made it VALU-bound: 25 M weights x 256 row blocks at 16384 rows).  The two
 // waves of a SIMD are in different groups: the first converts the next step's
 // tile before its MFMAs, the second after, and the MFMAs have the higher wave
-// priority, so one's conversion (VALU) runs beside the other's MFMAs (both
-// after: 791 us for 16384 rows of 12352 features; no priority: 871).
-// 16384 rows x 12352 x 2048: 1638 -> 740 us, 1.12 PFLOP/s; the library's fp16
-// product of that shape takes 731.  The matrix cores are busy 56% of the
-// cycles, at a clock that falls as they get busier (1.7 GHz of 2.4).
+// priority, so one's conversion (VALU) runs beside the other's MFMAs (256 x 256,
+// both after: 791 us for 16384 rows of 12352 features; no priority: 871).
 //
-// Every result is one accumulator over K in order, whatever the tile, and the
-// rows and K alone choose the kernel, so grouped and separate calls agree bit
-// for bit.
+// SUMS: the sums of the K-split kernel's four waves, bit for bit, so that a
+// launch is free to take either kernel: the chunks in its waves' order (c, c +
+// 4, ..), each wave's sum in one accumulator and added to the total when it is
+// complete, its K order inside a chunk (MFMA s takes the 8-element pieces 2 g +
+// s) and the same MFMA per piece.  The total takes as many registers again, so
+// a wave's tile is 64 x 64 at most: 256 x 128, one workgroup per CU (16384 rows x
+// 12352 x 2048: 924 us), or 128 x 128, two (1027).
+// Without SUMS: one accumulator over K in order, 64 x 128 a wave (24 operand
+// reads for 64 MFMAs against 32) in tiles of 256 x 256: 788 us on the same box,
+// 1.05 PFLOP/s; the matrix cores are busy 56% of the cycles, at a clock that
+// falls as they get busier (1.7 GHz of 2.4).
 //
 // LDS half: x, then weights, as 16-byte entries (8 K of one row): entry
 // (row tile rt, K piece q = 0 .. 7, row r) at (rt * 8 + q) * 16 + (r ^ swz(q)),
 // swz(q) = q for x and q & 6 for weights.  A store's 8 lanes (one row x 8
 // pieces of x; 2 rows x 4 alternate pieces of weights) hit 8 entries distinct
-// modulo 8.  An operand read takes lanes 0-3, 12-15 of one piece with lanes
-// 4-11 of the next in one pass, so two such pieces' XORs may differ in bits 0
-// and 1 only (bits 2 and 3 together): with x's q ^ 8 (q & 1) the kernel ran
-// 871 us against 758, 544 conflict cycles a step.
-template <int BM, int BN, int WM, int WN, bool XB>
-__global__ __launch_bounds__(64 * (BM / WM) * (BN / WN)) void linear_fp8_mm_kernel(const LinearArgs a) {
+// modulo 8.  An operand read takes lanes 0-3, 12-15 of one lane group with lanes
+// 4-11 of the next in one pass, so the XORs of two such groups' pieces (0, 1 and
+// 2, 3, whatever s) may differ in bits 0 and 1 only (bits 2 and 3 together):
+// with x's q ^ 8 (q & 1) the kernel ran 871 us against 758, 544 conflict cycles
+// a step.
+template <int BM, int BN, int WM, int WN, bool XB, bool SUMS>
+__global__ __launch_bounds__(64 * (BM / WM) * (BN / WN), 2) void linear_fp8_mm_kernel(const LinearArgs a) {
   using F16 = Kv16<RIA_DT_F16>;
   constexpr int NW = (BM / WM) * (BN / WN), NT = 64 * NW;
   constexpr int MT = WM / 16, FT = WN / 16;      // row and feature tiles of a wave
@@ -943,13 +948,13 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN)) void linear_fp8_mm_kern
   int x_rd[2], w_rd[2];
 #pragma unroll
   for (int s = 0; s < 2; ++s) {
-    const int q = 4 * s + g4;
+    const int q = SUMS ? 2 * g4 + s : 4 * s + g4;
     x_rd[s] = (wm * MT * 8 + q) * 16 + (n16 ^ swz_x(q));
     w_rd[s] = BM * 8 + (wn * FT * 8 + q) * 16 + (n16 ^ swz_w(q));
   }
   u32x4 xs[XL], ws[WL];
   float sc[WL];
-  auto load = [&](int c) __attribute__((always_inline)) {  // step c into registers (past the last: the last again)
+  auto load = [&](int c) __attribute__((always_inline)) {  // chunk c into registers (past the last: the last again)
     const int ko = min(c, steps - 1) * kKsChunk;
 #pragma unroll
     for (int i = 0; i < XL; ++i)
@@ -1002,27 +1007,57 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN)) void linear_fp8_mm_kern
     }
   };
   const bool first = wave < NW / 2;
-  load(0);
+  constexpr int kSums = 4;  // waves of the K-split kernel
+  auto next = [&](int c) { return !SUMS || c + kSums < steps ? c + (SUMS ? kSums : 1) : c % kSums + 1; };
+  f32x4 tot[SUMS ? FT : 1][SUMS ? MT : 1];
+  if constexpr (SUMS) {
+#pragma unroll
+    for (int f = 0; f < FT; ++f)
+#pragma unroll
+      for (int r = 0; r < MT; ++r) tot[f][r] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  int c = 0, c1 = next(c), c2 = next(c1);  // the chunk of this step and of the two after it
+  load(c);
   store(0);
-  load(1);
+  load(c1);
   lds_barrier();
-  for (int c = 0; c < steps; ++c) {
-    const bool more = c + 1 < steps;
+  for (int t = 0; t < steps; ++t) {
+    const bool more = t + 1 < steps;
     if (first && more) {
-      store((c + 1) & 1);
-      load(c + 2);
+      store((t + 1) & 1);
+      load(c2);
     }
     __builtin_amdgcn_sched_barrier(0);
     __builtin_amdgcn_s_setprio(1);
-    compute(c & 1);
+    compute(t & 1);
     __builtin_amdgcn_s_setprio(0);
     __builtin_amdgcn_sched_barrier(0);
     if (!first && more) {
-      store((c + 1) & 1);
-      load(c + 2);
+      store((t + 1) & 1);
+      load(c2);
     }
+    if constexpr (SUMS) {
+      if (c + kSums >= steps) {  // the last chunk of one sum
+#pragma unroll
+        for (int f = 0; f < FT; ++f)
+#pragma unroll
+          for (int r = 0; r < MT; ++r) {
+            tot[f][r] += acc[f][r];
+            acc[f][r] = f32x4{0.f, 0.f, 0.f, 0.f};
+          }
+      }
+    }
+    c = c1;
+    c1 = c2;
+    c2 = next(c2);
     lds_barrier();
   }
+  auto result = [&](int f, int r) -> const f32x4& {
+    if constexpr (SUMS)
+      return tot[f][r];
+    else
+      return acc[f][r];
+  };
   // F.linear's fp16 results, staged row by row in LDS (both halves are dead),
   // then stored as whole 8-feature pieces of rows.
   constexpr int kPitch = BN + 8;  // fp16 values of a staged row
@@ -1041,7 +1076,7 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN)) void linear_fp8_mm_kern
 #pragma unroll
         for (int r = 0; r < MT; ++r)
           *reinterpret_cast<u32x2*>(stg + (wm * WM % kPartRows + 16 * r + n16) * kPitch + wn * WN + 16 * f + 4 * g4) =
-              u32x2{F16::pack2(acc[f][r][0], acc[f][r][1]), F16::pack2(acc[f][r][2], acc[f][r][3])};
+              u32x2{F16::pack2(result(f, r)[0], result(f, r)[1]), F16::pack2(result(f, r)[2], result(f, r)[3])};
     }
     __syncthreads();
     constexpr int kPieces = kPartRows * BN / 8;
@@ -1137,50 +1172,76 @@ static void launch_ks(const LinearArgs& a, KsShape s, dim3 grid, hipStream_t st)
     launch_ks_k<2, 2, 6, XB>(a, grid, st);
 }
 
-// Tiles of the many-row kernel (BM rows x BN features).
-struct MmShape {
+// The kernel of one launch and its tile (bm rows x bn features).
+enum class LinKind { kGemv, kSplit, kManySums, kMany, kStream };
+struct LinPlan {
+  LinKind kind;
   int bm, bn;
 };
-// Fewest rows that take the many-row kernel.  A tile walks K serially, where
-// the K-split kernel's four waves share it, so the line rises with K: at K =
-// 2048, 256 rows of a layer's input projections 40.3 -> 31.7 us, 384 57.7 ->
-// 43.1 (300 rows 41.1 and 43.3); at K = 4096 and 2048 features, 1536 rows 60.1
-// -> 54.5 and 1024 rows 34.9 against 53.9.  The features do not enter: grouped
-// and separate calls must take the same kernel.
-static int mm_min_rows(int k) { return k <= 2048 ? 193 : 1345 * (k / 128) / 32; }
 
-static void launch_mm(const LinearArgs& a, MmShape s, bool xb, dim3 grid, hipStream_t st) {
-  if (s.bm == 256) {
-    if (xb)
-      hipLaunchKernelGGL((linear_fp8_mm_kernel<256, 256, 64, 128, true>), grid, dim3(512), 0, st, a);
-    else
-      hipLaunchKernelGGL((linear_fp8_mm_kernel<256, 256, 64, 128, false>), grid, dim3(512), 0, st, a);
-  } else {
-    if (xb)
-      hipLaunchKernelGGL((linear_fp8_mm_kernel<128, 128, 64, 64, true>), grid, dim3(256), 0, st, a);
-    else
-      hipLaunchKernelGGL((linear_fp8_mm_kernel<128, 128, 64, 64, false>), grid, dim3(256), 0, st, a);
-  }
+template <bool XB>
+static void launch_mm(const LinearArgs& a, const LinPlan& p, dim3 grid, hipStream_t st) {
+  if (p.kind == LinKind::kMany)
+    hipLaunchKernelGGL((linear_fp8_mm_kernel<256, 256, 64, 128, XB, false>), grid, dim3(512), 0, st, a);
+  else if (p.bm == 256)
+    hipLaunchKernelGGL((linear_fp8_mm_kernel<256, 128, 64, 64, XB, true>), grid, dim3(512), 0, st, a);
+  else
+    hipLaunchKernelGGL((linear_fp8_mm_kernel<128, 128, 64, 64, XB, true>), grid, dim3(256), 0, st, a);
 }
 
-// 256 x 256 tiles, one workgroup per CU, or 128 x 128, two: by the time of the
-// launch's rounds at K = 2048 on MI355X (a round of 256 x 256 tiles 54 us; of
-// 128 x 128 ones 30 with one per CU, 43 with two).  640 rows of a layer's
-// input projections take 47 us in small tiles and 53 in large, 777 rows 72 and
-// 58, 16384 rows 1035 and 740.
-static MmShape choose_mm(int m, int count, const ria_fp8_proj* projs) {
+static int64_t lin_tiles(int m, int count, const ria_fp8_proj* projs, int bm, int bn) {
+  int64_t t = 0;
+  for (int j = 0; j < count; ++j) t += (projs[j].n + bn - 1) / bn;
+  return t * ((m + bm - 1) / bm);
+}
+
+// Whether a projection takes the 256 x 256 tiles of one accumulator, whose bits
+// are not those of the other kernels: by its own rows and features alone (a
+// group of both kinds takes two launches), so grouped and separate calls agree
+// bit for bit.  From 2^25 results on, two such tiles for each CU, a projection
+// alone gains more than the rest of its group loses in a launch of its own:
+// 16384 rows of a layer's 12352 input projections (K = 2048) 779 us in two
+// launches, 944 in 256 x 128 tiles, 786 all in 256 x 256; 4096 rows 240, 274 and
+// 230.
+static bool takes_mm256(int m, int n) { return n >= 256 && static_cast<int64_t>(m) * n >= (int64_t(1) << 25); }
+
+// K-split tiles or the tiles that give the same bits: the least time by rounds
+// of tiles over the CUs, in microseconds at K = 2048 on MI355X (other K scale all
+// of them).  K-split: the shape whose busiest CU moves the fewest bytes, (rounds
+// of workgroups over the CUs) x (x + weight bytes of one tile), 17 us a round of
+// 64 x 128.  128 x 128: 30 us a round with one tile per CU, 46 with two; 256 x
+// 128: 38.  So the K-split kernel runs while its tiles fill the CUs once, m n =
+// 2^21 results (256 rows of 512 features 6.0 us, 24.6 in 128 x 128 tiles even of
+// one accumulator; of 8192 features 17.6 and 25), and the others past that: 12352 features x 193 rows 40.3
+// -> 33.4 us, 512 rows 78 -> 41.5, 640 rows 84 -> 50, 1024 rows 141 -> 80, 2048
+// rows 258 -> 156, while 300 rows stay (43.5, and 45.5 in 128 x 128 tiles).  Up to
+// 192 rows the larger tiles would be half padding.  Fewer than 512 features are
+// three columns of tiles at most, for which x sets the time: 100000 rows x 32
+// 80 us, 102 in 256 x 128 tiles; 12000 rows x 256 at K = 16384 212 and 231.
+static LinPlan plan_split(int m, int count, const ria_fp8_proj* projs) {
   const int64_t cus = device_cus();
-  int64_t t256 = 0, t128 = 0;
-  for (int j = 0; j < count; ++j) {
-    t256 += (projs[j].n + 255) / 256;
-    t128 += (projs[j].n + 127) / 128;
+  auto rounds = [&](int64_t tiles) { return (tiles + cus - 1) / cus; };
+  int64_t best = -1;
+  LinPlan plan{};
+  for (const KsShape s : kKsShapes) {
+    const int64_t cost = rounds(lin_tiles(m, count, projs, 16 * s.rt, 16 * s.ct)) * (32 * s.rt + 16 * s.ct);
+    if (best < 0 || cost < best) {
+      best = cost;
+      plan = LinPlan{LinKind::kSplit, 16 * s.rt, 16 * s.ct};
+    }
   }
-  t256 *= (m + 255) / 256;
-  t128 *= (m + 127) / 128;
-  const int64_t rest = t128 % (2 * cus);
-  const int64_t large = (t256 + cus - 1) / cus * 54;
-  const int64_t small = t128 / (2 * cus) * 43 + (rest == 0 ? 0 : rest <= cus ? 30 : 43);
-  return small < large ? MmShape{128, 128} : MmShape{256, 256};
+  int features = 0;
+  for (int j = 0; j < count; ++j) features += projs[j].n;
+  if (m < 193 || features < 512) return plan;
+  double us = best * (17.0 / 256);
+  const int64_t t128 = lin_tiles(m, count, projs, 128, 128), rest = t128 % (2 * cus);
+  const double us128 = static_cast<double>(t128 / (2 * cus) * 46 + (rest == 0 ? 0 : rest <= cus ? 30 : 46));
+  if (us128 < us) {
+    us = us128;
+    plan = LinPlan{LinKind::kManySums, 128, 128};
+  }
+  if (38.0 * rounds(lin_tiles(m, count, projs, 256, 128)) < us) plan = LinPlan{LinKind::kManySums, 256, 128};
+  return plan;
 }
 
 static bool lin_dtype_ok(int dt) { return dt == RIA_DT_BF16 || dt == RIA_DT_F16 || dt == RIA_DT_F32; }
@@ -1213,8 +1274,93 @@ extern "C" int ria_dequant_fp8(int64_t rows, int cols, const void* weight, const
   return check_launch("ria_dequant_fp8");
 }
 
-// Validates and launches one group of projections of the same x (shared by
-// ria_linear_fp8 and ria_linear_fp8_group; `who` names the entry point in errors).
+// Launches one group of projections of the same x, validated, by one kernel.
+static int launch_group(const char* who, const LinPlan& p, int m, int k, const void* x, int x_dtype,
+                        int64_t x_row_stride, int count, const ria_fp8_proj* projs, void* stream, const float* norm_w,
+                        float norm_eps, int norm_dtype) {
+  // Streaming kernel: workgroups of mt rows x 16 ct output features.  A
+  // workgroup reads its mt rows of x (from L2) and its weights through the
+  // CU's L1, whose misses in flight bound the rate, so the shape is the one
+  // whose busiest CU moves the fewest bytes: (workgroups per CU) x (x bytes
+  // + weight bytes of one workgroup); ties go to more workgroups.
+  int ct = 1, mt = kLinRows;
+  if (p.kind != LinKind::kStream && p.kind != LinKind::kGemv) {
+    ct = p.bn / 16;
+    mt = p.bm;
+  } else if (p.kind == LinKind::kStream) {
+    const int cus = device_cus();
+    int64_t best = -1, best_wgs = 0;
+    for (const int r : {kLinRows, kLinRows / 2})
+      for (const int c : {1, 2, 4}) {
+        int64_t wgs = 0;
+        for (int j = 0; j < count; ++j) wgs += (projs[j].n + 16 * c - 1) / (16 * c);
+        wgs *= (m + r - 1) / r;
+        const int64_t per_cu = (wgs + cus - 1) / cus * ((int64_t)std::min(r, m) * k * 2 + (int64_t)16 * c * k);
+        if (best < 0 || per_cu < best || (per_cu == best && wgs > best_wgs)) {
+          best = per_cu;
+          best_wgs = wgs;
+          ct = c;
+          mt = r;
+        }
+      }
+  }
+  LinearArgs a{};
+  a.x = x;
+  a.x_stride = x_row_stride;
+  a.m = m;
+  a.k = k;
+  a.count = count;
+  a.mt = mt;
+  a.norm_w = norm_w;
+  a.norm_eps = norm_eps;
+  a.norm_dtype = norm_dtype;
+  int tile = 0;
+  for (int j = 0; j < count; ++j) {
+    const ria_fp8_proj& q = projs[j];
+    a.p[j] = Fp8Proj{static_cast<const uint8_t*>(q.weight), q.scale_inv, q.y, q.y_row_stride, q.n, q.y_dtype, q.y_add,
+                     tile};
+    tile += (q.n + 16 * ct - 1) / (16 * ct);
+  }
+  a.tiles = tile;
+  const int64_t mblocks = p.kind == LinKind::kGemv ? 1 : (m + mt - 1) / mt;
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  if (p.kind == LinKind::kMany || p.kind == LinKind::kManySums) {
+    const int64_t wgs = (mblocks * tile + 7) / 8 * 8;
+    if (m > 65535LL * 64 || wgs > 0x7fffffff) return set_error(RIA_ERR_INVALID, "%s: too many rows", who);
+    if (x_dtype == RIA_DT_BF16)
+      launch_mm<true>(a, p, dim3(static_cast<unsigned>(wgs)), st);
+    else
+      launch_mm<false>(a, p, dim3(static_cast<unsigned>(wgs)), st);
+    return check_launch(who);
+  }
+  if (mblocks > 65535) return set_error(RIA_ERR_INVALID, "%s: too many rows", who);
+  const dim3 grid(static_cast<unsigned>(tile), static_cast<unsigned>(mblocks));
+  if (norm_w) {
+    launch_gemv<RIA_DT_F32, true>(a, grid, st);
+  } else if (p.kind == LinKind::kGemv) {
+    if (x_dtype == RIA_DT_F16)
+      launch_gemv<RIA_DT_F16>(a, grid, st);
+    else if (x_dtype == RIA_DT_BF16)
+      launch_gemv<RIA_DT_BF16>(a, grid, st);
+    else
+      launch_gemv<RIA_DT_F32>(a, grid, st);
+  } else if (p.kind == LinKind::kSplit) {
+    const KsShape shape{p.bm / 16, p.bn / 16};
+    if (x_dtype == RIA_DT_BF16)
+      launch_ks<true>(a, shape, grid, st);
+    else
+      launch_ks<false>(a, shape, grid, st);
+  } else if (x_dtype == RIA_DT_BF16) {
+    launch_linear<RIA_DT_BF16>(a, ct, grid, st);
+  } else {
+    launch_linear<RIA_DT_F32>(a, ct, grid, st);
+  }
+  return check_launch(who);
+}
+
+// Validates one group of projections of the same x and picks its kernels
+// (shared by ria_linear_fp8 and ria_linear_fp8_group; `who` names the entry
+// point in errors).
 static int linear_group(const char* who, int m, int k, const void* x, int x_dtype, int64_t x_row_stride, int count,
                         const ria_fp8_proj* projs, void* stream, const float* norm_w = nullptr, float norm_eps = 0.f,
                         int norm_dtype = RIA_DT_F16) {
@@ -1257,104 +1403,24 @@ static int linear_group(const char* who, int m, int k, const void* x, int x_dtyp
     if (norm_dtype != RIA_DT_BF16 && norm_dtype != RIA_DT_F16)
       return set_error(RIA_ERR_INVALID, "%s: fused norm rounds to bf16 or fp16", who);
   }
-  // Streaming kernel: workgroups of mt rows x 16 ct output features.  A
-  // workgroup reads its mt rows of x (from L2) and its weights through the
-  // CU's L1, whose misses in flight bound the rate, so the shape is the one
-  // whose busiest CU moves the fewest bytes: (workgroups per CU) x (x bytes
-  // + weight bytes of one workgroup); ties go to more workgroups.
-  int ct = 1, mt = kLinRows;
-  MmShape mm_shape{};
-  // K-split kernel (fp16 or bf16 x): the tile shape whose busiest CU moves the
-  // fewest bytes, (rounds of workgroups over the CUs) x (x + weight bytes of
-  // one tile)
-  bool ks = !gemv && (x_dtype == RIA_DT_F16 || x_dtype == RIA_DT_BF16) && (int64_t)m * x_row_stride < (int64_t(1) << 31);
+  auto launch = [&](const LinPlan& p, int n, const ria_fp8_proj* list) {
+    return launch_group(who, p, m, k, x, x_dtype, x_row_stride, n, list, stream, norm_w, norm_eps, norm_dtype);
+  };
+  if (gemv) return launch(LinPlan{LinKind::kGemv, 0, 0}, count, projs);
+  bool ks = (x_dtype == RIA_DT_F16 || x_dtype == RIA_DT_BF16) && (int64_t)m * x_row_stride < (int64_t(1) << 31);
   for (int j = 0; j < count; ++j) ks = ks && (int64_t)projs[j].n * k < (int64_t(1) << 31);
-  KsShape ks_shape = kKsShapes[0];
-  const bool mm = ks && m >= mm_min_rows(k);
-  if (mm) {
-    mm_shape = choose_mm(m, count, projs);
-    ct = mm_shape.bn / 16;
-    mt = mm_shape.bm;
-  } else if (ks) {
-    const int cus = device_cus();
-    int64_t best = -1;
-    for (const KsShape s : kKsShapes) {
-      int64_t wgs = 0;
-      for (int j = 0; j < count; ++j) wgs += (projs[j].n + 16 * s.ct - 1) / (16 * s.ct);
-      wgs *= (m + 16 * s.rt - 1) / (16 * s.rt);
-      const int64_t cost = (wgs + cus - 1) / cus * ((int64_t)k * (32 * s.rt + 16 * s.ct));
-      if (best < 0 || cost < best) {
-        best = cost;
-        ks_shape = s;
-      }
-    }
-    ct = ks_shape.ct;
-    mt = 16 * ks_shape.rt;
-  } else if (!gemv) {
-    const int cus = device_cus();
-    int64_t best = -1, best_wgs = 0;
-    for (const int r : {kLinRows, kLinRows / 2})
-      for (const int c : {1, 2, 4}) {
-        int64_t wgs = 0;
-        for (int j = 0; j < count; ++j) wgs += (projs[j].n + 16 * c - 1) / (16 * c);
-        wgs *= (m + r - 1) / r;
-        const int64_t per_cu = (wgs + cus - 1) / cus * ((int64_t)std::min(r, m) * k * 2 + (int64_t)16 * c * k);
-        if (best < 0 || per_cu < best || (per_cu == best && wgs > best_wgs)) {
-          best = per_cu;
-          best_wgs = wgs;
-          ct = c;
-          mt = r;
-        }
-      }
-  }
-  LinearArgs a{};
-  a.x = x;
-  a.x_stride = x_row_stride;
-  a.m = m;
-  a.k = k;
-  a.count = count;
-  a.mt = mt;
-  a.norm_w = norm_w;
-  a.norm_eps = norm_eps;
-  a.norm_dtype = norm_dtype;
-  int tile = 0;
+  if (!ks) return launch(LinPlan{LinKind::kStream, 0, 0}, count, projs);
+  ria_fp8_proj split[kLinGroup], many[kLinGroup];
+  int nsplit = 0, nmany = 0;
   for (int j = 0; j < count; ++j) {
-    const ria_fp8_proj& q = projs[j];
-    a.p[j] = Fp8Proj{static_cast<const uint8_t*>(q.weight), q.scale_inv, q.y, q.y_row_stride, q.n, q.y_dtype, q.y_add,
-                     tile};
-    tile += (q.n + 16 * ct - 1) / (16 * ct);
-  }
-  a.tiles = tile;
-  const int64_t mblocks = gemv ? 1 : (m + mt - 1) / mt;
-  if (mm) {
-    const int64_t wgs = (mblocks * tile + 7) / 8 * 8;
-    if (m > 65535LL * 64 || wgs > 0x7fffffff) return set_error(RIA_ERR_INVALID, "%s: too many rows", who);
-    launch_mm(a, mm_shape, x_dtype == RIA_DT_BF16, dim3(static_cast<unsigned>(wgs)), static_cast<hipStream_t>(stream));
-    return check_launch(who);
-  }
-  if (mblocks > 65535) return set_error(RIA_ERR_INVALID, "%s: too many rows", who);
-  const dim3 grid(static_cast<unsigned>(tile), static_cast<unsigned>(mblocks));
-  hipStream_t st = static_cast<hipStream_t>(stream);
-  if (norm_w) {
-    launch_gemv<RIA_DT_F32, true>(a, grid, st);
-  } else if (gemv) {
-    if (x_dtype == RIA_DT_F16)
-      launch_gemv<RIA_DT_F16>(a, grid, st);
-    else if (x_dtype == RIA_DT_BF16)
-      launch_gemv<RIA_DT_BF16>(a, grid, st);
+    if (takes_mm256(m, projs[j].n))
+      many[nmany++] = projs[j];
     else
-      launch_gemv<RIA_DT_F32>(a, grid, st);
-  } else if (ks) {
-    if (x_dtype == RIA_DT_BF16)
-      launch_ks<true>(a, ks_shape, grid, st);
-    else
-      launch_ks<false>(a, ks_shape, grid, st);
-  } else if (x_dtype == RIA_DT_BF16) {
-    launch_linear<RIA_DT_BF16>(a, ct, grid, st);
-  } else {
-    launch_linear<RIA_DT_F32>(a, ct, grid, st);
+      split[nsplit++] = projs[j];
   }
-  return check_launch(who);
+  // the launch whose limit on the rows is the lowest first: a group is refused whole
+  const int rc = nsplit ? launch(plan_split(m, nsplit, split), nsplit, split) : RIA_OK;
+  return rc == RIA_OK && nmany ? launch(LinPlan{LinKind::kMany, 256, 256}, nmany, many) : rc;
 }
 
 extern "C" int ria_linear_fp8(int m, int n, int k, const void* x, int x_dtype, int64_t x_row_stride,

@@ -237,3 +237,36 @@ def test_many_row_kernel(gpu, m, ns, k, xdt):
         y = base.clone()
         K.linear_fp8_group(x, [(w, s)], out=[y], accumulate=[True])
         assert torch.equal(y, base + ys[j].float())
+
+
+@pytest.mark.parametrize("xdt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("m,n,k", [
+    (193, 512, 2048), (256, 2048, 4096),  # few tiles: the K-split kernel
+    (257, 8192, 128), (321, 8208, 4224),  # 128 x 128 tiles, fewer chunks of K than sums, a feature tile of 16
+    (450, 12352, 384), (513, 9216, 2048),  # 256 x 128 tiles, a ragged last chunk of the sums, one row past a tile
+])
+def test_rows_do_not_depend_on_the_call(gpu, m, n, k, xdt):
+    """A prompt's projection against the same rows in calls of 96 to 160 rows:
+    whatever kernel and tile a call takes below 2^25 results, the same bits."""
+    announce(f"linear_fp8 rows of a call: M={m} N={n} K={k} x {xdt}")
+    w, s = (t.to(gpu) for t in W.fp8_block_weight(900 + k, n, k))
+    x = torch.randn((m, k), generator=torch.Generator().manual_seed(910 + m)).to(xdt).to(gpu)
+    whole = K.linear_fp8(x, w, s)
+    assert torch.equal(whole, torch.cat([K.linear_fp8(part, w, s) for part in x.chunk((m + 159) // 160)]))
+
+
+@pytest.mark.parametrize("xdt", [torch.bfloat16, torch.float16])
+def test_group_of_two_launches(gpu, xdt):
+    """A group whose projections take different kernels (2048 features of 16400
+    rows are more than 2^25 results): the bits of separate calls, each within
+    1.5x of the fp32-accumulated product's error."""
+    m, ns, k = 16400, [512, 2048, 32], 256
+    announce(f"linear_fp8_group in two launches: M={m} N={ns} K={k} x {xdt}")
+    proj = [tuple(t.to(gpu) for t in W.fp8_block_weight(930 + j, n, k)) for j, n in enumerate(ns)]
+    x = torch.randn((m, k), generator=torch.Generator().manual_seed(940)).to(xdt).to(gpu)
+    for y, (w, s) in zip(K.linear_fp8_group(x, proj), proj):
+        assert torch.equal(y, K.linear_fp8(x, w, s))
+        w16, x16 = K.dequant_fp8(w, s, torch.float16), x.to(torch.float16)
+        exact = x16.double() @ w16.double().t()
+        e_got, e_ref = ((t.double() - exact).abs().max().item() for t in (y, (x16.float() @ w16.float().t()).half()))
+        assert e_got <= 1.5 * e_ref + 1e-6, (e_got, e_ref)
