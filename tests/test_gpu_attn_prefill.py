@@ -268,3 +268,26 @@ def test_attn_prefill_32_token_blocks(gpu, length, hq, hkv, staged):
     first = K.attn_prefill(q[:n], k[:n], v[:n], gate[:n], kv.k[0], kv.v[0], kv.page_table[0], start=0, **kw)
     assert float((out[t0:] - last).abs().max()) <= tol
     assert float((out[:n] - first).abs().max()) <= tol
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("length,start,token", [(6048, 0, 3000), (6035, 0, 6033), (6048, 13, 2995), (6048, 16, 2987)])
+def test_attn_prefill_infinite_value_reaches_no_earlier_block(gpu, length, start, token):
+    """A value of infinity: the queries before its block of 16 tokens, which
+    the causal mask keeps from it, give the bits they give without it, also
+    where two blocks of 16 share a workgroup."""
+    announce(f"attn_prefill: infinite V at token {token} of {length} after {start}")
+    q, k, v, gate = (x.to(gpu) for x in _inputs(31, length, dtype=torch.float16))
+    k0, v0 = (x.to(gpu) for x in _inputs(32, max(start, 1), dtype=torch.float16)[1:3])
+    outs = []
+    for value in (1.0, float("inf")):
+        v[token] = value
+        kv = _cache(gpu, start + length, dtype=torch.float16)
+        inv = rope_inv_freq(10_000_000.0, 64).to(gpu)
+        if start:
+            K.kv_append_seq(k0, v0, kv.k[0], kv.v[0], kv.page_table[0], start=0, inv_freq=inv)
+        outs.append(_run(gpu, kv, q, k, v, gate, start))
+    before = token // 16 * 16
+    assert bool(torch.isfinite(outs[0]).all())
+    assert torch.equal(outs[1][:before], outs[0][:before])
+    assert bool((~torch.isfinite(outs[1][token:])).any(-1).all())
