@@ -38,6 +38,7 @@
 //     groups with permlane swaps;
 //   * the gated result leaves through LDS so the output stores are coalesced;
 //   * query blocks are scheduled from the last (most keys) to the first.
+#include <float.h>
 #include <math.h>
 #include <algorithm>
 
@@ -90,8 +91,7 @@ struct PrefillAttnArgs {
 
 // Pieces.  The keys of a query block are split every `chunk` 32-key blocks,
 // as far as a piece's first key is visible to the block's first query (so
-// every column of every piece has a finite max); the last piece takes the
-// rest.  Piece s exists for the query blocks qb >= first_query_block(s).  A
+// every column of every piece sees a key); the last piece takes the rest.  Piece s exists for the query blocks qb >= first_query_block(s).  A
 // launch lists the pieces by s, each s from the last query block down, and
 // both kernels find a piece's index by the same counts.
 __host__ __device__ inline int first_query_block(int s, int chunk, int start, int nqb, int qt) {
@@ -295,7 +295,9 @@ __global__ __launch_bounds__(kPrefillThreads) __attribute__((amdgpu_waves_per_eu
   for (int c = 0; c < NC; ++c) {
 #pragma unroll
     for (int dt = 0; dt < NO; ++dt) o[c][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
-    m_run[c] = -INFINITY;
+    // below every score, and finite: a block or piece whose scores are all -inf
+    // (infinite keys) then weighs 0 instead of exp2(-inf + inf)
+    m_run[c] = -FLT_MAX;
     l_run[c] = 0.f;
   }
   constexpr uint32_t kOne2 = KVT == RIA_DT_F16 ? 0x3C003C00u : 0x3F803F80u;  // two 16-bit 1.0
@@ -407,8 +409,7 @@ __global__ __launch_bounds__(kPrefillThreads) __attribute__((amdgpu_waves_per_eu
       }
       if (__any(mloc > m_run[c] + 8.0f)) {
         const float mx = swap_max(swap_max(mloc, true), false);
-        // m_run is finite from the first block on (the piece's first key is
-        // visible to every column), so masked scores give exp2(-inf) = 0
+        // m_run is finite, so masked scores give exp2(-inf) = 0
         const bool grow = mx > m_run[c] + 8.0f;
         const float m_new = grow ? mx : m_run[c];
         const float alpha = __builtin_amdgcn_exp2f(m_run[c] - m_new);  // 0 on the first block, where o and l are 0

@@ -291,3 +291,28 @@ def test_attn_prefill_infinite_value_reaches_no_earlier_block(gpu, length, start
     assert bool(torch.isfinite(outs[0]).all())
     assert torch.equal(outs[1][:before], outs[0][:before])
     assert bool((~torch.isfinite(outs[1][token:])).any(-1).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("length,start", [(500, 7900), (64, 4000)])
+def test_attn_prefill_split_with_infinite_keys(gpu, length, start):
+    """Resident keys that score -inf for every query, whole pieces of the split
+    among them, weigh nothing in the merge: the unsplit launch's result."""
+    announce(f"attn_prefill split: {length} after {start}, keys 40 .. {start - 1} score -inf")
+    _, k0, v0, _ = _inputs(41, start, dtype=torch.float32)
+    q, k, v, gate = (x.to(gpu) for x in _inputs(42, length, dtype=torch.float32))
+    q[..., 100] = q[..., 100].abs() + 0.5  # past the rotary dims
+    k0[40:, :, 100] = float("-inf")
+    inv = rope_inv_freq(10_000_000.0, 64).to(gpu)
+    kv = _cache(gpu, start + length, dtype=torch.float16)
+    K.kv_append_seq(k0.to(gpu), v0.to(gpu), kv.k[0], kv.v[0], kv.page_table[0], start=0, inv_freq=inv)
+    need = K.prefill_attn_workspace_bytes(length, 16, 2, start, True)
+    assert need > 0, "a split case"
+    ws = torch.empty(need, dtype=torch.uint8, device=gpu)
+    args = (q, k, v, gate, kv.k[0], kv.v[0], kv.page_table[0])
+    kw = dict(start=start, inv_freq=inv, scale=SCALE)
+    whole = K.attn_prefill(*args, **kw)
+    split = K.attn_prefill(*args, **kw, workspace=ws)
+    assert bool(torch.isfinite(whole).all())
+    vmax = float(max(v.abs().max(), v0.abs().max()))
+    assert float((split - whole).abs().max()) <= 4 * vmax * 2.0 ** -11 + 1e-5  # fp16 probabilities of both
