@@ -76,3 +76,38 @@ def test_engine_prefill_then_decode(gpu):
                                                               att["gate"][t, r:r + 1], t)
             assert_act_close(got_att[r][t], want[0], f"row {r} attention token {t}")
         assert_state_close(st.linear_states[0, r].cpu()[None], s.linear[0], f"row {r} final state")
+
+
+def test_rows_prefilled_on_two_streams(gpu):
+    """Two prompts from empty rows, their layers issued in turn on two streams: the serial result's bits."""
+    announce("engine: rows prefilled with 1500 and 1100 tokens on two streams, then serially")
+    prompts, layers = [1500, 1100], 3
+    params = W.gdn_layer_params(71)
+    cw, alog, dtb = (params[n].to(gpu) for n in ("conv_weight", "A_log", "dt_bias"))
+    g = torch.Generator(device=gpu)
+    g.manual_seed(72)
+    rows = [[torch.randn((n, *shape), generator=g, device=gpu).to(dt) for shape, dt in (
+        ((W.CONV_DIM,), torch.bfloat16), ((32,), torch.float32), ((32,), torch.float32), ((16, 256), torch.bfloat16),
+        ((2, 256), torch.bfloat16), ((2, 256), torch.bfloat16), ((16, 256), torch.bfloat16))] for n in prompts]
+
+    def run(streams):
+        st = BatchedAttentionState(2, 1600, num_linear_layers=layers, num_full_layers=layers, device=gpu,
+                                   prefill_segment_tokens=512)
+        st.set_positions([0, 0])
+        for row, n in enumerate(prompts):
+            st.begin_prefill(row, n)
+        torch.cuda.synchronize()
+        outs = []
+        for layer in range(layers):
+            for row, (mixed, a, b, q, k, v, gate) in enumerate(rows):
+                with torch.cuda.stream(streams[row]):
+                    outs.append(st.linear_prefill(layer, row, mixed, cw, a, b, gate_mode=nat.RIA_GATE_RAW, A_log=alog,
+                                                  dt_bias=dtb))
+                    outs.append(st.full_prefill(layer, row, q, k, v, gate))
+        torch.cuda.synchronize()
+        return outs + [st.linear_states, st.conv_rings, st.kv.k, st.kv.v]
+
+    serial = torch.cuda.current_stream()
+    want = run([serial, serial])
+    got = run([torch.cuda.Stream(), torch.cuda.Stream()])
+    assert all(torch.equal(x, y) for x, y in zip(got, want))
