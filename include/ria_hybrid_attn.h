@@ -62,7 +62,7 @@
 extern "C" {
 #endif
 
-#define RIA_ABI_VERSION 5
+#define RIA_ABI_VERSION 6
 
 enum ria_dtype { RIA_DT_BF16 = 0, RIA_DT_F16 = 1, RIA_DT_F32 = 2 };
 

@@ -15,7 +15,7 @@ from pathlib import Path
 
 LIB_ENV = "RIA_HIP_LIB"
 DEFAULT_LIB = Path(__file__).resolve().parent / "_lib" / "libria_hip.so"
-ABI_VERSION = 5
+ABI_VERSION = 6
 
 RIA_DT_BF16 = 0
 RIA_DT_F16 = 1
@@ -221,13 +221,16 @@ def load() -> ctypes.CDLL:
             f"or `make -C router-ia_amd/csrc`, or point {LIB_ENV} at a built libria_hip.so"
         )
     lib = ctypes.CDLL(str(path))
+    # the version before the entry points: another version may lack some of them
+    if not hasattr(lib, "ria_abi_version"):
+        raise NativeLibraryError(f"{path} has no ABI version, expected {ABI_VERSION}")
+    version = lib.ria_abi_version()
+    if version != ABI_VERSION:
+        raise NativeLibraryError(f"{path} has ABI version {version}, expected {ABI_VERSION}")
     for name, (restype, argtypes) in SIGNATURES.items():
         fn = getattr(lib, name)
         fn.restype = restype
         fn.argtypes = argtypes
-    version = lib.ria_abi_version()
-    if version != ABI_VERSION:
-        raise NativeLibraryError(f"{path} has ABI version {version}, expected {ABI_VERSION}")
     _LIB = lib
     return lib
 

@@ -53,6 +53,18 @@ def test_abi_version_and_host_side_validation() -> None:
     assert lib.ria_attn_decode_workspace_bytes(1, 16, 2, 64, 64) > 0
 
 
+@pytest.mark.parametrize("exports", [{"ria_abi_version": lambda: 5}, {}], ids=["an earlier version", "no version"])
+def test_library_of_another_version_is_refused(monkeypatch, tmp_path, exports) -> None:
+    """A version-5 build lacks entry points of this one: refused by its version, not by a missing name."""
+    stale = tmp_path / "libria_hip.so"
+    stale.touch()
+    monkeypatch.setenv(nat.LIB_ENV, str(stale))
+    monkeypatch.setattr(nat, "_LIB", None)
+    monkeypatch.setattr(nat.ctypes, "CDLL", lambda path: type("Library", (), {k: staticmethod(f) for k, f in exports.items()}))
+    with pytest.raises(nat.NativeLibraryError, match="ABI version"):
+        nat.load()
+
+
 @pytest.mark.parametrize("ctx,expect", [([4097], 64), ([8193] * 32, 512), ([32768] * 128, 3072)])
 def test_split_heuristic(ctx, expect) -> None:
     from router_ia import kernels as K
