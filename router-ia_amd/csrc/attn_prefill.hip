@@ -664,6 +664,9 @@ static void launch_prefill(const PrefillAttnArgs& a, const int32_t* pt, int kv_d
 // all are busy) of 16 tokens with fp16 keys 1.05, 1.15, of 32 tokens 1.36,
 // 1.65, of 16 tokens with bf16 hi + lo operands 1.8; prologue and epilogue 14
 // per 16 tokens; combine 6 + one per 40 pieces of 16 tokens.
+// A split has to promise 3%: of 644 prompts of other lengths, positions and head
+// counts those promised less (2500 tokens after 13, 0.8%: 145 us whole, 166 cut;
+// 300 after 700 with 8 KV heads, 1%: 66 and 71) were the only ones it slowed down.
 struct PrefillPlan {
   int qt;          // tokens of a query block
   int chunk;       // 0: unsplit
@@ -672,8 +675,8 @@ struct PrefillPlan {
 static PrefillPlan plan_prefill(int length, int start, int num_kv_heads, bool fp16_keys, int max_pieces) {
   const int cus = device_cus();
   const int most = ((start + length - 1) / kPageTokens + 2) / 2;  // key blocks of the last query block
-  PrefillPlan best{};
-  double best_cost = -1;
+  PrefillPlan best[2]{};  // whole query blocks; split
+  double best_cost[2] = {-1, -1};
   for (int qt = 16; qt <= (fp16_keys ? 32 : 16); qt += 16) {
     const int nqb = (length + qt - 1) / qt;
     const double block = !fp16_keys ? 1.8 : qt == 16 ? 1.05 : 1.36;
@@ -694,13 +697,14 @@ static PrefillPlan plan_prefill(int length, int start, int num_kv_heads, bool fp
         if (pieces > cus) cost = std::max(cost, work / cus + longest / 4);
         cost += 6.0 + pieces * qt / 640.0;
       }
-      if (best_cost < 0 || cost < best_cost) {
-        best_cost = cost;
-        best = PrefillPlan{qt, chunk, pieces};
+      const int split = k > 1;
+      if (best_cost[split] < 0 || cost < best_cost[split]) {
+        best_cost[split] = cost;
+        best[split] = PrefillPlan{qt, chunk, pieces};
       }
     }
   }
-  return best;
+  return best_cost[1] >= 0 && best_cost[1] < 0.97 * best_cost[0] ? best[1] : best[0];
 }
 
 static int64_t partial_bytes(const PrefillPlan& p, int group) {

@@ -216,3 +216,13 @@ def test_gdn_decode_ex_and_window_conv_host_validation() -> None:
     assert rc == 1 and b"aligned" in lib.ria_last_error()
     rc = lib.ria_conv1d_window_step(1, 8192, fake, 0, 4096, fake, fake, fake, fake, 2, None)
     assert rc == 1 and b"x_row_stride" in lib.ria_last_error()
+
+
+def test_prefill_split_is_left_out_where_it_promises_little() -> None:
+    """Prompts measured slower with their keys split (2500 tokens after 13, 300 after 700 with 8 KV heads) run whole."""
+    from router_ia import kernels as K
+
+    assert K.prefill_attn_workspace_bytes(2500, 16, 2, 13, False) == 0
+    assert K.prefill_attn_workspace_bytes(300, 64, 8, 700, False) == 0
+    assert K.prefill_attn_workspace_bytes(500, 16, 2, 12000, False) > 0
+    assert K.prefill_attn_workspace_bytes(1000, 16, 2, 0, True) > 0
