@@ -316,3 +316,64 @@ def test_attn_prefill_split_with_infinite_keys(gpu, length, start):
     assert bool(torch.isfinite(whole).all())
     vmax = float(max(v.abs().max(), v0.abs().max()))
     assert float((split - whole).abs().max()) <= 4 * vmax * 2.0 ** -11 + 1e-5  # fp16 probabilities of both
+
+
+def _assert_same_but_rounding(got, want, vmax, fp16_keys):
+    """Two launches whose query blocks or pieces differ: the probabilities' rounding about different maxima
+    (2^-11 relative with fp16 keys, 2^-16 hi + lo, in products and normaliser of both), then each output's own
+    rounding to a 16-bit type (half a unit in the last place of both)."""
+    got, want, dt = got.float(), want.float(), want.dtype
+    ulp = {torch.float32: 0.0, torch.float16: 2.0 ** -10, torch.bfloat16: 2.0 ** -7}[dt]
+    tol = 4 * vmax * (2.0 ** -11 if fp16_keys else 2.0 ** -16) + 1e-5
+    assert bool(((got - want).abs() <= tol + ulp * torch.maximum(got.abs(), want.abs())).all())
+
+
+def _norms(gpu, seed):
+    g = torch.Generator().manual_seed(seed)
+    return {n: (0.1 * torch.randn(256, generator=g)).to(gpu) for n in ("q_norm_weight", "k_norm_weight")}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("length,start,pages", [(1000, 0, torch.bfloat16), (500, 7900, torch.bfloat16),
+                                                (500, 7900, torch.float16), (33, 1024, torch.float16)])
+def test_attn_prefill_split_16_bit_activations_and_norms(gpu, length, start, pages, dtype):
+    """16-bit q, k, v and gate with q_norm and k_norm, in pieces of 16 and 32 tokens, against the unsplit launch."""
+    staged = start == 0
+    announce(f"attn_prefill split with norms: {length} after {start}, {dtype} over {pages} pages")
+    _, k0, v0, _ = _inputs(51, max(start, 1), dtype=dtype)
+    q, k, v, gate = (x.to(gpu) for x in _inputs(52 + length, length, dtype=dtype))
+    inv = rope_inv_freq(10_000_000.0, 64).to(gpu)
+    kv = _cache(gpu, start + length, dtype=pages)
+    if start:
+        K.kv_append_seq(k0.to(gpu), v0.to(gpu), kv.k[0], kv.v[0], kv.page_table[0], start=0, inv_freq=inv)
+    fp16 = staged or pages == torch.float16
+    need = K.prefill_attn_workspace_bytes(length, 16, 2, start, fp16)
+    assert need > 0, "a split case"
+    args = (q, k, v, gate, kv.k[0], kv.v[0], kv.page_table[0])
+    stage = torch.empty(K.prefill_stage_bytes(length, 2), dtype=torch.uint8, device=gpu) if staged else None
+    kw = dict(start=start, inv_freq=inv, scale=SCALE, stage=stage, **_norms(gpu, 53))
+    whole = K.attn_prefill(*args, **kw)
+    pages_whole = kv.k.clone(), kv.v.clone()
+    split = K.attn_prefill(*args, **kw, workspace=torch.full((need,), 0xFF, dtype=torch.uint8, device=gpu))
+    assert torch.equal(kv.k, pages_whole[0]) and torch.equal(kv.v, pages_whole[1])
+    _assert_same_but_rounding(split, whole, float(max(v.abs().max(), v0.abs().max())), fp16)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+def test_attn_prefill_32_token_blocks_with_norms(gpu, dtype):
+    """q_norm in a 32-token block's prologue: a long prompt's first and last tokens against blocks of 16."""
+    length, n = 6031, 70
+    announce(f"attn_prefill 32-token blocks with norms: L={length}, {dtype}, fp16 pages")
+    q, k, v, gate = (x.to(gpu) for x in _inputs(61, length, dtype=dtype))
+    kv = _cache(gpu, length, dtype=torch.float16)
+    kw = dict(inv_freq=rope_inv_freq(10_000_000.0, 64).to(gpu), scale=SCALE, **_norms(gpu, 62))
+    cache = (kv.k[0], kv.v[0], kv.page_table[0])
+    out = K.attn_prefill(q, k, v, gate, *cache, start=0, **kw)
+    t0 = length - n
+    last = K.attn_prefill(q[t0:], k[t0:], v[t0:], gate[t0:], *cache, start=t0, **kw)
+    first = K.attn_prefill(q[:n], k[:n], v[:n], gate[:n], *cache, start=0, **kw)
+    vmax = float(v.abs().max())
+    _assert_same_but_rounding(out[t0:], last, vmax, True)
+    _assert_same_but_rounding(out[:n], first, vmax, True)

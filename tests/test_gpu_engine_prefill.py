@@ -16,6 +16,7 @@ from conftest import announce
 from helpers import assert_act_close, assert_state_close
 from oracle import qwen36_cpu as O
 from router_ia import _native as nat
+from router_ia import kernels as K
 from router_ia import workloads as W
 from router_ia.batched_state import BatchedAttentionState
 
@@ -111,3 +112,31 @@ def test_rows_prefilled_on_two_streams(gpu):
     want = run([serial, serial])
     got = run([torch.cuda.Stream(), torch.cuda.Stream()])
     assert all(torch.equal(x, y) for x, y in zip(got, want))
+
+
+def test_full_prefill_splits_short_prompts(gpu):
+    """A prompt of 1000 tokens and a turn of 300 after it through the engine, which splits their keys, against
+    unsplit launches over a second engine's pages: the same pages, outputs within the probabilities' rounding
+    (fp16 keys in the first prompt: 2^-11 relative, bf16 hi + lo after it: 2^-16, in products and normaliser of
+    both launches)."""
+    announce("engine: full_prefill of 1000 + 300 tokens with split keys")
+    g = torch.Generator(device=gpu)
+    g.manual_seed(81)
+    one, other = (BatchedAttentionState(1, 1400, num_linear_layers=0, num_full_layers=1, device=gpu,
+                                        page_shuffle_seed=3) for _ in range(2))
+    start = 0
+    for n, u in ((1000, 2.0 ** -11), (300, 2.0 ** -16)):
+        assert K.prefill_attn_workspace_bytes(n, 16, 2, start, start == 0) > 0, "a split case"
+        q, k, v, gate = (torch.randn((n, h, 256), generator=g, device=gpu) for h in (16, 2, 2, 16))
+        for st in (one, other):
+            st.begin_prefill(0, n)
+        got = one.full_prefill(0, 0, q, k, v, gate)
+        stage = torch.empty(K.prefill_stage_bytes(n, 2), dtype=torch.uint8, device=gpu) if start == 0 else None
+        want = K.attn_prefill(q, k, v, gate, *other.kv.layer(0), other.kv.page_table[0], start=start,
+                              inv_freq=other.inv_freq, scale=other.scale, stage=stage)
+        assert torch.equal(one.kv.k, other.kv.k) and torch.equal(one.kv.v, other.kv.v)
+        # values of every key so far are standard normal, below 6
+        assert float((got - want).abs().max()) <= 4 * 6 * u + 1e-5
+        for st in (one, other):
+            st.end_prefill(0, n)
+        start += n
