@@ -22,12 +22,12 @@ class _Calls:
         self.stream, self.capturing, self.held = 1, False, []
         monkeypatch.setattr(K, "gdn_prefill", self._record)
         monkeypatch.setattr(K, "attn_prefill", self._record)
-        monkeypatch.setattr(K, "_stream", lambda device: self.stream)
+        monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda device: self.stream, raising=False)
         monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: self.capturing)
         st = self.st = object.__new__(BatchedAttentionState)  # only what the prefill methods read
         st.device = torch.device("cpu")
         st.num_k_heads, st.num_v_heads, st.num_q_heads, st.num_kv_heads = 16, 32, 16, 2
-        st.prefill_segment_tokens, st._prefill_scratch = 4096, {}
+        st.prefill_segment_tokens, st._prefill_scratch, st._device_index = 4096, {}, 0
         st.linear_states = st.conv_rings = torch.zeros((1, 2, 1))
         st.inv_freq, st.scale, st._host_seen = None, 1.0, seen
         st.kv = SimpleNamespace(layer=lambda i: (None, None), page_table=[None, None], dtype=torch.bfloat16)
