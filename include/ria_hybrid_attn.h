@@ -449,8 +449,11 @@ int ria_attn_prefill_staged(int length, int num_q_heads, int num_kv_heads,
  * chosen for a prompt (0: not split; fp16_keys: nonzero when the attention
  * reads fp16 keys, from the stage or an fp16 cache).  A workspace (16-byte
  * aligned) that is null or smaller runs unsplit.  The pages are those of
- * ria_attn_prefill_phase bit for bit, the outputs equal up to the order of the
- * fp32 sums.
+ * ria_attn_prefill_phase bit for bit.  The outputs are those of the unsplit
+ * launch but for the order of the fp32 sums and the rounding of the softmax's
+ * probabilities, which each piece rounds about its own running maximum: before
+ * their own rounding they differ within 4 * 2^-11 of the largest |v| with
+ * fp16 keys, 4 * 2^-16 with bf16 pages (hi + lo pairs).
  */
 int64_t ria_attn_prefill_workspace_bytes(int length, int num_q_heads, int num_kv_heads, int32_t start_pos,
                                          int fp16_keys);
@@ -651,10 +654,12 @@ int ria_kv_gather(int batch, int num_kv_heads,
  * rounded to fp16 (F.linear's fp16 output) and stored as y_dtype.  x [m, k]
  * of x_dtype (converted to fp16 like `.to(float16)`), y [m, n].  n a multiple
  * of 16, k of 128; x and weight 16-byte aligned, x row stride a multiple of 8.
- * Built for decode-sized m (one weight pass per 128 rows of x); k up to 32768.
+ * Decode batches read a weight once per 128 rows of x, prompts dequantise it
+ * once per 128 or 256; k up to 32768.
  *
- * ria_linear_fp8_group: 1 to 4 such projections of the same x in one launch,
- * each with its own n, weight, scales, y and y dtype.  It replaces
+ * ria_linear_fp8_group: 1 to 4 such projections of the same x in one launch
+ * (two where some have m n of 2^25 and more and some not), each with its own n,
+ * weight, scales, y and y dtype.  It replaces
  * the reference's run of F.linear calls on one normed hidden state: DeltaNet
  * in_proj_qkv / in_proj_z / in_proj_a / in_proj_b (qwen36_attention_cache.py:
  * 232-247, 268) and attention q_proj / k_proj / v_proj (:295-301); results

@@ -163,14 +163,6 @@ __global__ __launch_bounds__(256) void kv_append_kernel(AppendArgs a) {
   a.v_cache[(tile * kAttnHeadDim + d) * kPageTokens + off] = Kv16<KVT>::from_f32(vv);
 }
 
-// A prompt's append (one sequence, token i at position and slot
-// pos_scalar + i), one workgroup per (page, KV head): thread d owns dim d of
-// the page's 16 tokens and puts each through kv_append_kernel's arithmetic
-// (the same sums of squares, k_norm, RoPE and rounding), so the pages get
-// the same bits.  A page the prompt fills leaves as 16-byte stores: K
-// through an LDS copy of the tile (each 16-byte piece is 8 dims of one
-// token), V^T as each dim's 32-byte row; the first and last pages keep the
-// tokens outside the prompt (per-token stores).
 // wave_sum of 16 values at once, the same sums in the same order (xor 32, 16,
 // 8, 4, 2, 1): each of the first four steps adds the halves of two values in
 // one go, half the lanes keeping one and half the other, so 16 sums take 17
@@ -200,6 +192,14 @@ __device__ __forceinline__ float wave_sum16(const float (&x)[16]) {
   return add_rn(v, __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xB1, 0xf, 0xf, true)));  // quad lane ^ 1
 }
 
+// A prompt's append (one sequence, token i at position and slot
+// pos_scalar + i), one workgroup per (page, KV head): thread d owns dim d of
+// the page's 16 tokens and puts each through kv_append_kernel's arithmetic
+// (the same sums of squares, k_norm, RoPE and rounding), so the pages get
+// the same bits.  A page the prompt fills leaves as 16-byte stores: K
+// through an LDS copy of the tile (each 16-byte piece is 8 dims of one
+// token), V^T as each dim's 32-byte row; the first and last pages keep the
+// tokens outside the prompt (per-token stores).
 template <int KT, int VT, int KVT>
 __global__ __launch_bounds__(256) void kv_append_page_kernel(AppendArgs a) {
   const int d = threadIdx.x, lane = d & 63, w = d >> 6;

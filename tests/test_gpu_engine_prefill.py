@@ -140,3 +140,42 @@ def test_full_prefill_splits_short_prompts(gpu):
         for st in (one, other):
             st.end_prefill(0, n)
         start += n
+
+
+def test_recorded_prefill_replays_beside_eager_prompts(gpu):
+    """One row's two layers in a HIP graph, replayed with longer eager prompts of the other row on the same stream
+    between (they grow the eager scratch): every replay gives the eager bits."""
+    announce("engine: recorded prefill of 700 tokens, replayed three times beside eager prompts of 900 .. 1500")
+    n = 700
+    params = W.gdn_layer_params(91)
+    cw, alog, dtb = (params[x].to(gpu) for x in ("conv_weight", "A_log", "dt_bias"))
+    g = torch.Generator(device=gpu)
+    g.manual_seed(92)
+    mixed = torch.randn((1500, W.CONV_DIM), generator=g, device=gpu).to(torch.bfloat16)
+    a, b = (torch.randn((1500, 32), generator=g, device=gpu) for _ in range(2))
+    q, k, v, gate = (torch.randn((1500, h, 256), generator=g, device=gpu).to(torch.bfloat16) for h in (16, 2, 2, 16))
+    st = BatchedAttentionState(2, 1600, num_linear_layers=1, num_full_layers=1, device=gpu)
+    st.set_positions([0, 0])
+    st.begin_prefill(0, n)
+    st.begin_prefill(1, 1500)
+
+    def run(row, m):
+        return [st.linear_prefill(0, row, mixed[:m], cw, a[:m], b[:m], gate_mode=nat.RIA_GATE_RAW, A_log=alog,
+                                  dt_bias=dtb), st.full_prefill(0, row, q[:m], k[:m], v[:m], gate[:m])]
+
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        want = [x.clone() for x in run(0, n)]
+        state = st.linear_states[0, 0].clone()
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            outs = run(0, n)
+        for m in (900, 1200, 1500):
+            run(1, m)
+            st.linear_states[0, 0].zero_()
+            st.conv_rings[0, 0].zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert all(torch.equal(x, y) for x, y in zip(outs, want))
+            assert torch.equal(st.linear_states[0, 0], state)
