@@ -207,10 +207,12 @@ def test_linear_fp8_group_normed_host_checks(gpu):
 @pytest.mark.parametrize("xdt", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("m,ns,k", [
     (193, [8192, 32], 2048),            # fewest rows, 128 x 128 tiles, a 32-wide projection
-    (255, [48, 272], 128),              # two steps of K, features that end inside a tile
-    (777, [8192, 4096, 32, 32], 2048),  # 256 x 256 tiles, 9 rows past a tile
-    (4097, [272, 1040], 384),           # one row past a tile, three scale blocks of K
-    (1345, [512], 4096),                # fewest rows at K = 4096
+    (255, [48, 272], 128),              # few features: the K-split kernel, fewer chunks of K than its waves
+    (777, [8192, 4096, 32, 32], 2048),  # 128 x 128 tiles, two to a CU, 9 rows past a tile
+    (4097, [272, 1040], 384),           # 256 x 128 tiles, one row past a tile, three scale blocks of K
+    (1345, [512], 4096),                # few tiles at K = 4096: the K-split kernel
+    (16400, [2064], 384),               # 256 x 256 tiles, 16 rows and 16 features past a tile
+    (131089, [272, 16], 128),           # 256 x 256 tiles of two steps of K, and 16 features in the other launch
 ])
 def test_many_row_kernel(gpu, m, ns, k, xdt):
     """Prompt-sized calls against the exact product of the same fp16 operands
